@@ -111,3 +111,29 @@ def test_overlapped_swap_step_matches_sequential_moves():
     assert np.array_equal(_np(pool).reshape(expect.shape), expect)
     with pytest.raises(ValueError):
         mover.swap([1], host_out[:1], [1], host_in[:1])
+
+
+@pytest.mark.parametrize("planes,row_bytes,n", [
+    (1, 16, 1),                    # one vector, one workgroup of the eight launched
+    (1, 16 * 1024, 7),             # one full piece per row, 7 pieces over 8 XCDs
+    (3, 16 * 1024 + 16, 3),        # a second piece of one vector; 18 pieces
+    (5, 3 * 16 * 1024 - 16, 13),   # a last piece one vector short; 195 pieces
+])
+def test_device_moves_at_piece_and_xcd_edges(planes, row_bytes, n):
+    g = torch.Generator().manual_seed(7)
+    pool = torch.randint(0, 256, (1, planes, 2 * n + 1, row_bytes), generator=g,
+                         dtype=torch.uint8).to(DEV)
+    ids = torch.randperm(2 * n + 1, generator=g).tolist()
+    src, dst = ids[:n], ids[n:2 * n]
+    mover = BlockMover(pool)
+    before = pool.clone()
+    print(f"[blocks] edges planes={planes} row={row_bytes} n={n}", flush=True)
+    items = mover.gather(src)
+    assert torch.equal(items, before[:, :, src].movedim(2, 0))
+    expect = before.clone()
+    expect[:, :, dst] = before[:, :, src]
+    mover.copy(src, dst)
+    assert torch.equal(pool, expect)
+    expect[:, :, src] = items.movedim(0, 2).flip(2)
+    mover.scatter(items.flip(0), src)
+    assert torch.equal(pool, expect)
