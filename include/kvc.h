@@ -534,6 +534,29 @@ int kvc_qk_norm_rope_store(const void* q, int64_t q_stride_t, int64_t q_stride_h
                            void* v_cache, int64_t num_slots, const void* slot_mapping,
                            int slot_index_bytes, kvc_stream_t stream);
 
+/* ---------------------------------------------------------------------------
+ * Inputs of a captured decode step.
+ * ------------------------------------------------------------------------- */
+
+/* Refreshes the static buffers a captured decode step reads, in one launch
+ * (nanovllm/engine/model_runner.py:864-869).  Row r < batch of layer l of
+ * q / k / v (q_row_bytes / kv_row_bytes at src + l*layer_stride +
+ * r*row_stride, bytes, all multiples of 16 and 16-byte aligned) goes to row r
+ * of the dense [layers][dst_rows] destination; rows batch .. bucket - 1 are
+ * zeroed.  slots_dst / lens_dst [bucket] take slot_mapping / context_lens
+ * (int32 or int64 by index bytes), then scratch_slot / 1; row r of tables_dst
+ * [dst_rows, dst_cols] takes block_tables' bt_cols entries (row stride
+ * bt_stride elements), everything else scratch_block. */
+int kvc_stage_decode(const void* q, int64_t q_layer_stride, int64_t q_row_stride, const void* k,
+                     int64_t k_layer_stride, int64_t k_row_stride, const void* v,
+                     int64_t v_layer_stride, int64_t v_row_stride, int64_t q_row_bytes,
+                     int64_t kv_row_bytes, int64_t layers, int64_t batch, int64_t bucket,
+                     int64_t dst_rows, const void* slot_mapping, int slot_index_bytes,
+                     const void* context_lens, int lens_index_bytes, const int32_t* block_tables,
+                     int64_t bt_stride, int64_t bt_cols, void* q_dst, void* k_dst, void* v_dst,
+                     int32_t* slots_dst, int32_t* lens_dst, int32_t* tables_dst, int64_t dst_cols,
+                     int32_t scratch_slot, int32_t scratch_block, kvc_stream_t stream);
+
 #ifdef __cplusplus
 }
 #endif

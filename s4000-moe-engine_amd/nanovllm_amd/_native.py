@@ -98,6 +98,9 @@ SIGNATURES = {
                                       _I64, _I64, _I64, _I64, _P, _INT, _P, _P, _F32,
                                       _P, _I64, _P, _I64, _I64, _P, _I64, _I64, _P, _P,
                                       _I64, _P, _INT, _P]),
+    "kvc_stage_decode": (_INT, [_P, _I64, _I64, _P, _I64, _I64, _P, _I64, _I64, _I64, _I64, _I64,
+                                _I64, _I64, _I64, _P, _INT, _P, _INT, _P, _I64, _I64, _P, _P, _P,
+                                _P, _P, _P, _I64, _INT, _INT, _P]),
 }
 
 _lock = threading.Lock()

@@ -8,16 +8,19 @@ Follows the engine's decode graph protocol (nanovllm/engine/model_runner.py:
   the pool's reserved scratch block: slot_mapping = scratch slot,
   context_lens = 1, block-table rows = the scratch block id.  They write and
   read only that block, never a live one;
-* graph inputs are static buffers refreshed before each replay; the padding
-  fills and copies run eagerly, outside the graph.  Padded q/k/v rows are
-  zeros, so the padded rows' appends (all to the one scratch slot) store the
-  same bytes whichever lands last.
+* graph inputs are static buffers refreshed before each replay, outside the
+  graph, by one staging launch (inputs of other forms than the step's own go
+  through torch's copies and fills).  Padded q/k/v rows are zeros, so the
+  padded rows' appends (all to the one scratch slot) store the same bytes
+  whichever lands last.
 
 What is captured is the path's part of a decode step, per layer:
 store_kvcache(k, v, k_cache, v_cache, slot_mapping) then the paged decode,
 as one paged_decode_append call (the append rides in the decode launch; a
 padded row's slot is position 0 of its scratch-block table row, as the fused
-append requires).  Nothing records a host synchronisation or a memset: loop
+append requires), which writes the runner's output buffer itself: a copy
+node per layer cost 4-5 us each on the replay's critical path.  Nothing
+records a host synchronisation or a memset: loop
 bounds come from the device context_lens, and the split-K workspace is taken
 from torch's caching allocator (the graph's private pool during capture).
 """
@@ -25,7 +28,8 @@ from __future__ import annotations
 
 import torch
 
-from ..kernels.paged_attention import paged_decode_append
+from .. import _native as nat
+from ..kernels.paged_attention import decode_append_into
 
 
 def default_buckets(max_bs: int) -> list[int]:
@@ -110,9 +114,9 @@ class DecodeGraphRunner:
         sm, cl, bt = self.slot_mapping[:bs], self.context_lens[:bs], self.block_tables[:bs]
         for layer in range(self.num_layers):
             kc, vc = self.k_caches[layer], self.v_caches[layer]
-            self.out[layer, :bs] = paged_decode_append(
-                self.q[layer, :bs], self.k[layer, :bs], self.v[layer, :bs], kc, vc, sm, bt, cl,
-                self.scale)
+            decode_append_into(
+                self.out[layer, :bs], self.q[layer, :bs], self.k[layer, :bs], self.v[layer, :bs],
+                kc, vc, sm, bt, cl, self.scale)
 
     def capture(self) -> None:
         """Capture every bucket, small first (model_runner.py:1169-1175): a
@@ -136,14 +140,44 @@ class DecodeGraphRunner:
                 return b
         raise ValueError(f"batch {bs} exceeds the largest bucket {max(self.buckets)}")
 
-    def run(self, q, k, v, slot_mapping, context_lens, block_tables) -> torch.Tensor:
-        """One replay, after the runner's fence (asynchronous block moves
-        issued so far are ordered before the replay's pool reads and
-        appends)."""
-        bs = q.size(1)
-        if self.fence is not None:
-            self.fence()
-        b = self.bucket_of(bs)
+    def _stageable(self, bs: int, q, k, v, slot_mapping, context_lens, block_tables) -> bool:
+        """Inputs the staging launch reads as they are: bf16 rows whose heads
+        are dense and 16-byte aligned, int32 / int64 vectors, int32 tables,
+        all on the runner's device."""
+        for t, buf in ((q, self.q), (k, self.k), (v, self.v)):
+            if t.dtype != buf.dtype or t.device != buf.device or t.dim() != 4 \
+                    or t.size(0) != buf.size(0) or t.size(1) != bs or t.shape[2:] != buf.shape[2:] \
+                    or t.stride(3) != 1 or t.stride(2) != self.head_dim \
+                    or t.stride(0) % 8 or t.stride(1) % 8 or t.data_ptr() % 16:
+                return False
+        for t in (slot_mapping, context_lens):
+            if t.dtype not in (torch.int32, torch.int64) or t.device != self.q.device \
+                    or t.dim() != 1 or t.numel() != bs or not t.is_contiguous():
+                return False
+        t = block_tables
+        return (t.dtype == torch.int32 and t.device == self.q.device and t.dim() == 2
+                and t.size(0) == bs and t.size(1) <= self.block_tables.size(1)
+                and (t.stride(1) == 1 or t.size(1) <= 1))
+
+    def _stage(self, bs: int, b: int, q, k, v, slot_mapping, context_lens, block_tables) -> None:
+        """Bucket b's static buffers from a batch of bs rows."""
+        if bs > 0 and self.head_dim % 8 == 0 and self.q.element_size() == 2 \
+                and self._stageable(bs, q, k, v, slot_mapping, context_lens, block_tables):
+            nat.call(
+                "kvc_stage_decode",
+                q.data_ptr(), q.stride(0) * 2, q.stride(1) * 2,
+                k.data_ptr(), k.stride(0) * 2, k.stride(1) * 2,
+                v.data_ptr(), v.stride(0) * 2, v.stride(1) * 2,
+                self.num_heads * self.head_dim * 2, self.num_kv_heads * self.head_dim * 2,
+                self.num_layers, bs, b, self.max_bs,
+                slot_mapping.data_ptr(), slot_mapping.element_size(),
+                context_lens.data_ptr(), context_lens.element_size(),
+                block_tables.data_ptr(), block_tables.stride(0), block_tables.size(1),
+                self.q.data_ptr(), self.k.data_ptr(), self.v.data_ptr(),
+                self.slot_mapping.data_ptr(), self.context_lens.data_ptr(),
+                self.block_tables.data_ptr(), self.block_tables.size(1),
+                self.scratch_slot, self.scratch_block_id, nat.stream_of(self.q))
+            return
         self.q[:, :bs] = q
         self.k[:, :bs] = k
         self.v[:, :bs] = v
@@ -156,5 +190,15 @@ class DecodeGraphRunner:
         pad_decode_inputs(slot_mapping, context_lens, block_tables, self.slot_mapping[:b],
                           self.context_lens[:b], self.block_tables[:b], self.scratch_slot,
                           self.scratch_block_id)
+
+    def run(self, q, k, v, slot_mapping, context_lens, block_tables) -> torch.Tensor:
+        """One replay, after the runner's fence (asynchronous block moves
+        issued so far are ordered before the replay's pool reads and
+        appends)."""
+        bs = q.size(1)
+        if self.fence is not None:
+            self.fence()
+        b = self.bucket_of(bs)
+        self._stage(bs, b, q, k, v, slot_mapping, context_lens, block_tables)
         self.graphs[b].replay()
         return self.out[:, :bs]

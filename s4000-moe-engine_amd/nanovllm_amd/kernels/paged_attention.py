@@ -158,6 +158,14 @@ def paged_decode_append(q, key, value, k_cache, v_cache, slot_mapping, block_tab
     allows.  That needs the engine's decode slots (slot_mapping[b] is
     position context_lens[b] - 1 of row b, read by no other row).  Same
     results and pool contents as the two calls."""
+    return decode_append_into(None, q, key, value, k_cache, v_cache, slot_mapping, block_tables,
+                              context_lens, scale)
+
+
+def decode_append_into(output, q, key, value, k_cache, v_cache, slot_mapping, block_tables,
+                       context_lens, scale):
+    """paged_decode_append with the result written to `output` ([batch, heads,
+    128] bf16, unit inner stride; None: a new tensor), which is returned."""
     if q.ndim != 3 or key.ndim != 3 or value.shape != key.shape or k_cache.ndim != 4 \
             or v_cache.shape != k_cache.shape:
         raise ValueError("expected q=[batch,heads,dim], key/value=[batch,kv_heads,dim], "
@@ -190,9 +198,10 @@ def paged_decode_append(q, key, value, k_cache, v_cache, slot_mapping, block_tab
         slot_mapping = slot_mapping.to(torch.int32)
         sb = 4
     slot_mapping = slot_mapping.contiguous()
-    output = torch.empty_like(q)
-    if output.stride(2) != 1:
-        output = torch.empty(q.shape, dtype=q.dtype, device=q.device)
+    if output is None:
+        output = torch.empty_like(q)
+        if output.stride(2) != 1:
+            output = torch.empty(q.shape, dtype=q.dtype, device=q.device)
     if batch == 0:
         return output
     if _check_append_enabled():

@@ -162,3 +162,41 @@ def test_graph_replay_after_async_eviction_of_the_appended_block(deterministic_d
     flat = r.kv_cache.view(2, Lg, -1, KVH, 128)
     assert np.array_equal(bits(flat[0][:, slots.long().to(DEV)]), bits(k))
     assert np.array_equal(bits(flat[1][:, slots.long().to(DEV)]), bits(v))
+
+
+@pytest.mark.parametrize("heads,kvh", [(32, 4), (16, 2), (4, 1)])
+@pytest.mark.parametrize("bs,cols", [(1, 1), (4, MAXB), (5, 3), (15, 0), (16, MAXB)])
+@pytest.mark.parametrize("fused_view", [False, True])
+def test_staging_launch_equals_the_copies_and_fills(heads, kvh, bs, cols, fused_view):
+    """One staging launch against torch's copies and fills on the same buffers
+    (every byte, padding included), for dense rows and for views of a fused
+    [L, bs, (H + 2 KVH) * D] projection, int32 and int64 indices, table widths
+    0 .. the buffer's."""
+    dims = (heads, kvh)
+    pools = [torch.zeros(3, PAGE, kvh, 128, dtype=torch.bfloat16, device=DEV) for _ in range(L)]
+    runner = DecodeGraphRunner(pools, pools, heads, max_bs=16, max_blocks_per_seq=MAXB, scale=1.0)
+    g = torch.Generator().manual_seed(bs * 31 + cols)
+    qkv = torch.randn(L, bs, (heads + 2 * kvh) * 128, generator=g).to(torch.bfloat16).to(DEV)
+    q, k, v = qkv.split((heads * 128, kvh * 128, kvh * 128), dim=-1)
+    q, k, v = q.unflatten(-1, (heads, 128)), k.unflatten(-1, (kvh, 128)), v.unflatten(-1, (kvh, 128))
+    if not fused_view:
+        q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
+    wide = torch.int64 if bs % 2 else torch.int32
+    slots = torch.randint(0, 2 * PAGE, (bs,), generator=g).to(wide).to(DEV)
+    lens = torch.randint(1, 2 * PAGE, (bs,), generator=g).to(wide).to(DEV)
+    tables = torch.randint(-1, 3, (bs, MAXB), generator=g).to(torch.int32).to(DEV)[:, :cols]
+    b = runner.bucket_of(bs)
+    assert runner._stageable(bs, q, k, v, slots, lens, tables)
+    # a form the launch does not read (float32 q) takes the copies and fills
+    assert not runner._stageable(bs, q.float(), k, v, slots, lens, tables)
+    got = []
+    bufs = [runner.q, runner.k, runner.v, runner.slot_mapping, runner.context_lens,
+            runner.block_tables]
+    for q_in in (q, q.float()):
+        for t in bufs:
+            t.fill_(77)
+        print(f"[graph] stage heads={dims} bs={bs} cols={cols} view={fused_view}", flush=True)
+        runner._stage(bs, b, q_in, k, v, slots, lens, tables)
+        got.append([t.clone() for t in bufs])
+    for fast, plain in zip(*got):
+        assert torch.equal(fast, plain)
