@@ -2150,9 +2150,6 @@ struct I8LdsLayout<kI8Chan, kN> {
   static constexpr int kScales = kDummy + 1024;
   static constexpr int kBytes = kScales + 2048;
 };
-constexpr int cmax(int a, int b) { return a > b ? a : b; }
-constexpr int kLdsChan = cmax(I8LdsLayout<kI8Chan, 2>::kBytes,
-                              cmax(I8LdsLayout<kI8Chan, 4>::kBytes, I8LdsLayout<kI8Chan, 8>::kBytes));
 static_assert(4 * 16 * kI8MergePitch * 4 + 4 * 16 * (2 + 16) * 4 <= I8LdsLayout<kI8Chan, 8>::kSide,
               "per-channel merge block fits the stages");
 
@@ -3131,7 +3128,8 @@ __device__ void write_nan_rows(const AttnParams& p, int b, int kvg) {
 // kLds: 4 kv heads per workgroup staged through LDS, bf16
 // (decode_segment_lds: two stages in smem and smem1) or per-token-head int8
 // (decode_segment_lds_i8: a four-stage ring in smem); smem2 holds the query.
-template <int kEnc, bool kLds, bool kSteal = false, int kHeads = 4>
+// kSide: (per-channel LDS segments) the side pool's width, 2, 4 or 8.
+template <int kEnc, bool kLds, bool kSteal = false, int kHeads = 4, int kSide = 0>
 __device__ __forceinline__ void decode_sk_share(const AttnParams& p,
                                                 const int32_t* __restrict__ block_tables,
                                                 const int32_t* __restrict__ ctx_lens, int w,
@@ -3431,21 +3429,9 @@ __device__ __forceinline__ void decode_sk_share(const AttnParams& p,
     DecSeg sg;
     while (next_seg(sg)) {
       if constexpr (kI8Lds && kEnc == kI8Chan) {
-        const int32_t* bt = block_tables + int64_t(sg.b) * p.bt_stride;
-        switch (p.n_out_max) {
-          case 2:
-            decode_segment_lds_i8<kI8Chan, 2>(p, smem, smem2, bt, sg.b, sg.kvg, sg.ctx, sg.t0,
-                                              sg.t1, sg.split);
-            break;
-          case 8:
-            decode_segment_lds_i8<kI8Chan, 8>(p, smem, smem2, bt, sg.b, sg.kvg, sg.ctx, sg.t0,
-                                              sg.t1, sg.split);
-            break;
-          default:  // 4, or no side pool
-            decode_segment_lds_i8<kI8Chan, 4>(p, smem, smem2, bt, sg.b, sg.kvg, sg.ctx, sg.t0,
-                                              sg.t1, sg.split);
-            break;
-        }
+        decode_segment_lds_i8<kI8Chan, kSide>(p, smem, smem2,
+                                              block_tables + int64_t(sg.b) * p.bt_stride, sg.b,
+                                              sg.kvg, sg.ctx, sg.t0, sg.t1, sg.split);
       } else if constexpr (kI8Lds) {
         decode_segment_lds_i8<kI8Tok, 0>(p, smem, smem2,
                                          block_tables + int64_t(sg.b) * p.bt_stride, sg.b,
@@ -3471,14 +3457,26 @@ paged_decode_sk_kernel(AttnParams p, const int32_t* __restrict__ block_tables,
                        const int32_t* __restrict__ ctx_lens) {
   constexpr bool kBfLds = kLds && kEnc == kBF16;
   constexpr bool kI8Lds = kLds && kEnc == kI8Tok;
-  constexpr bool kChLds = kLds && kEnc == kI8Chan;
-  __shared__ __align__(16) char
-      smem[kBfLds ? kLdsStage : (kI8Lds ? kLdsI8 : (kChLds ? kLdsChan : kDecodeSmem))];
+  __shared__ __align__(16) char smem[kBfLds ? kLdsStage : (kI8Lds ? kLdsI8 : kDecodeSmem)];
   __shared__ __align__(16) char smem1[kBfLds ? kLdsStage : 16];
   __shared__ __align__(16) char smem2[kLds ? kLdsQ : 16];
   touch_kernel_args(int(sizeof(AttnParams) + 2 * sizeof(void*)));
   decode_sk_share<kEnc, kLds>(p, block_tables, ctx_lens, int(blockIdx.x), int(gridDim.x), smem,
                               smem1, smem2, StealArgs{});
+}
+
+// The per-channel int8 LDS decode, one kernel per side width: all three
+// widths in one kernel spilled (8 bytes of scratch a lane); 48 rows of
+// 1025-12007 keys, width 8: 79.6 us a call with one kernel, 79.0 us so.
+template <int kSide>
+__global__ void __launch_bounds__(kThreads)
+paged_decode_chan_kernel(AttnParams p, const int32_t* __restrict__ block_tables,
+                         const int32_t* __restrict__ ctx_lens) {
+  __shared__ __align__(16) char smem[I8LdsLayout<kI8Chan, kSide>::kBytes];
+  __shared__ __align__(16) char smem2[kLdsQ];
+  touch_kernel_args(int(sizeof(AttnParams) + 2 * sizeof(void*)));
+  decode_sk_share<kI8Chan, true, false, 4, kSide>(p, block_tables, ctx_lens, int(blockIdx.x),
+                                                  int(gridDim.x), smem, smem, smem2, StealArgs{});
 }
 
 // The bf16 LDS decode with 2 kv heads per workgroup.
@@ -5630,8 +5628,20 @@ int paged_decode_impl(const void* q, int64_t q_stride_b, int64_t q_stride_h, con
         // side rows); width 1 runs the register segment.
         if (hp.kvs_per_wg == 4 && hp.nslices == 1 && env_int("KVC_DECODE_LDS", 1) != 0 &&
             (head_n_out == nullptr || n_out_max >= 2)) {
-          paged_decode_sk_kernel<kI8Chan, true>
-              <<<sp.grid, kThreads, 0, st>>>(p, block_tables, context_lens);
+          switch (p.n_out_max) {
+            case 2:
+              paged_decode_chan_kernel<2>
+                  <<<sp.grid, kThreads, 0, st>>>(p, block_tables, context_lens);
+              break;
+            case 8:
+              paged_decode_chan_kernel<8>
+                  <<<sp.grid, kThreads, 0, st>>>(p, block_tables, context_lens);
+              break;
+            default:  // 4, or no side pool
+              paged_decode_chan_kernel<4>
+                  <<<sp.grid, kThreads, 0, st>>>(p, block_tables, context_lens);
+              break;
+          }
         } else {
           paged_decode_sk_kernel<kI8Chan, false>
               <<<sp.grid, kThreads, 0, st>>>(p, block_tables, context_lens);
