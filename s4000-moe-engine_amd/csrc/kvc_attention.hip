@@ -3945,17 +3945,26 @@ __device__ __forceinline__ void p2_load_chunk(PfItem& it, const int4* ctab, cons
 #define KVC_P2_ITEM_COST 6
 #endif
 constexpr int kP2ItemCost = KVC_P2_ITEM_COST;
+// With the residue product an item also reads its outlier dims' list and
+// folds the residues in at its end: four chunks of 300-512 tokens after 0-8192 keys took
+// 196 / 191 / 187.4 / 186.1 / 185.5 / 186.4 us a call at 6 / 7 / 8 / 9 / 10 / 12.
+#ifndef KVC_P2_ITEM_COST_RESIDUE
+#define KVC_P2_ITEM_COST_RESIDUE 10
+#endif
+constexpr int kP2ItemCostResidue = KVC_P2_ITEM_COST_RESIDUE;
 
 // Weighted tiles of query tiles [0, q) of chunk c.
+template <int kCost>
 __device__ __forceinline__ int p2_qcum(const ChunkGeo& c, int tpb, int q) {
-  return int(qtile_cum(c, tpb, q)) + kP2ItemCost * q;
+  return int(qtile_cum(c, tpb, q)) + kCost * q;
 }
 
 // The item after `it` (T = 0 past the last one), chunks read from the table.
+template <int kCost>
 __device__ __forceinline__ void p2_next_item(PfItem& it, const int4* ctab, const int32_t* cu_q,
                                              const int32_t* cu_k, int n_pre, int kvs_total,
                                              int nslices, int qtile) {
-  it.P += kP2ItemCost + it.T;
+  it.P += kCost + it.T;
   if (++it.qt == it.geo.ntq) {
     it.qt = 0;
     ++it.kvs;
@@ -3988,6 +3997,7 @@ __device__ __forceinline__ void prefill_sk2_share(const AttnParams& p,
                                                   const int32_t* __restrict__ block_tables,
                                                   const int v, const int G, char* lds,
                                                   int4* ctab) {
+  constexpr int kItemCost = kPLo ? kP2ItemCostResidue : kP2ItemCost;
   const unsigned long long t_start =
       p.wg_stamps != nullptr ? __builtin_amdgcn_s_memrealtime() : 0ull;
   auto stamp = [&]() {  // diagnostics: this workgroup's start and end
@@ -4015,7 +4025,7 @@ __device__ __forceinline__ void prefill_sk2_share(const AttnParams& p,
       const ChunkGeo c = chunk_geo(cu_q, cu_k, ci, qtile);
       if (c.ntq > 0) {
         tm = (c.sk + kTile - 1) / kTile;
-        t = kvs_total * p2_qcum(c, p.tpb, c.ntq);
+        t = kvs_total * p2_qcum<kItemCost>(c, p.tpb, c.ntq);
       }
       if (c0 == 0) {
         g_first = c;
@@ -4031,7 +4041,7 @@ __device__ __forceinline__ void prefill_sk2_share(const AttnParams& p,
   W = uniform(W);
   Tmax = uniform(Tmax);
   int S = max(p.sk_min_share, (W + G - 1) / G);
-  if (p.max_splits > 1) S = max(S, (Tmax + kP2ItemCost + p.max_splits - 2) / (p.max_splits - 1));
+  if (p.max_splits > 1) S = max(S, (Tmax + kItemCost + p.max_splits - 2) / (p.max_splits - 1));
   S = uniform(S);
   if (int64_t(w) * S >= W) {
     stamp();
@@ -4050,7 +4060,7 @@ __device__ __forceinline__ void prefill_sk2_share(const AttnParams& p,
         t = 0;
         if (c0 + L.lane < p.n_pre) {
           const ChunkGeo c = chunk_geo(cu_q, cu_k, c0 + L.lane, qtile);
-          if (c.ntq > 0) t = kvs_total * p2_qcum(c, p.tpb, c.ntq);
+          if (c.ntq > 0) t = kvs_total * p2_qcum<kItemCost>(c, p.tpb, c.ntq);
         }
       }
       const int inc = wave_scan_add(t);
@@ -4074,22 +4084,22 @@ __device__ __forceinline__ void prefill_sk2_share(const AttnParams& p,
     }
     it.i = ci;
     if (ci >= 64) pf_load_chunk(it, cu_q, cu_k, qtile);
-    const int per_kvs = p2_qcum(it.geo, p.tpb, it.geo.ntq);
+    const int per_kvs = p2_qcum<kItemCost>(it.geo, p.tpb, it.geo.ntq);
     int off = start - P;
     it.kvs = uniform(off / per_kvs);
     off -= it.kvs * per_kvs;
     int lo = 0, hi = it.geo.ntq - 1;
     while (lo < hi) {
       const int mid = (lo + hi + 1) >> 1;
-      if (p2_qcum(it.geo, p.tpb, mid) <= off) lo = mid; else hi = mid - 1;
+      if (p2_qcum<kItemCost>(it.geo, p.tpb, mid) <= off) lo = mid; else hi = mid - 1;
     }
     it.qt = uniform(lo);
     it.g = uniform(it.kvs / p.nslices);
     it.s = it.kvs - it.g * p.nslices;
-    it.P = uniform(P + it.kvs * per_kvs + p2_qcum(it.geo, p.tpb, it.qt));
+    it.P = uniform(P + it.kvs * per_kvs + p2_qcum<kItemCost>(it.geo, p.tpb, it.qt));
     it.T = qtile_tiles(it.geo, qtile, it.qt);
   }
-  int ct = max(0, start - it.P - kP2ItemCost);  // consumer's tile in `it`
+  int ct = max(0, start - it.P - kItemCost);  // consumer's tile in `it`
 
   // Tile loads: wave w issues loads w, w + 8, w + 16 of the 18 per tile (9 of
   // K, 9 of V; the six past 18 are zero loads into a dummy block).
@@ -4167,9 +4177,9 @@ __device__ __forceinline__ void prefill_sk2_share(const AttnParams& p,
     dma_to_lds_cached(rv, boff[2] + hv, w01 ? sb + dst2 : lds0 + kP2DummyOff);
     issued += kPfTileLoads;
     if (++pt == pi.T) {
-      p2_next_item(pi, ctab, cu_q, cu_k, p.n_pre, kvs_total, p.nslices, qtile);
+      p2_next_item<kItemCost>(pi, ctab, cu_q, cu_k, p.n_pre, kvs_total, p.nslices, qtile);
       pt = 0;
-      if (pi.P + kP2ItemCost < end) table_setup();
+      if (pi.P + kItemCost < end) table_setup();
     } else if constexpr (!kFresh) {
       poff += kTile;
       if (poff == p.page) {
@@ -4180,7 +4190,7 @@ __device__ __forceinline__ void prefill_sk2_share(const AttnParams& p,
       }
     }
   };
-  auto prod_live = [&]() { return pi.P + kP2ItemCost + pt < end; };
+  auto prod_live = [&]() { return pi.P + kItemCost + pt < end; };
 
   // This wave's query columns of item x into its LDS region: column c
   // (0..31: block c / 16, lane c % 16) at slots 17 c .. 17 c + 15; columns
@@ -4240,11 +4250,11 @@ __device__ __forceinline__ void prefill_sk2_share(const AttnParams& p,
     }
   };
   auto issue_next_q = [&]() {
-    const int nP = it.P + kP2ItemCost + it.T;  // span start of the item after `it`
-    if (nP + kP2ItemCost < end) {
+    const int nP = it.P + kItemCost + it.T;  // span start of the item after `it`
+    if (nP + kItemCost < end) {
       __builtin_amdgcn_s_waitcnt(kWaitLgkm0);
       PfItem nx = it;
-      p2_next_item(nx, ctab, cu_q, cu_k, p.n_pre, kvs_total, p.nslices, qtile);
+      p2_next_item<kItemCost>(nx, ctab, cu_q, cu_k, p.n_pre, kvs_total, p.nslices, qtile);
       issue_q(nx);
       q_mark = issued;
       q_for = nP;
@@ -4381,12 +4391,12 @@ __device__ __forceinline__ void prefill_sk2_share(const AttnParams& p,
   auto run_length = [&]() {
     const int mk = uniform(min_klim);
     const int unmasked = min(it.geo.sk >> 5, mk >= kTile - 1 ? ((mk - (kTile - 1)) >> 5) + 1 : 0);
-    const int r1 = min(min(it.T - 1, unmasked), end - 1 - (it.P + kP2ItemCost)) - ct;
-    const int r2 = min(pi.T - 1 - pt, end - (pi.P + kP2ItemCost + pt));
+    const int r1 = min(min(it.T - 1, unmasked), end - 1 - (it.P + kItemCost)) - ct;
+    const int r2 = min(pi.T - 1 - pt, end - (pi.P + kItemCost + pt));
     return uniform(max(0, min(r1, r2)));
   };
 
-  while (it.P + kP2ItemCost + ct < end) {
+  while (it.P + kItemCost + ct < end) {
     if (!first && ct != 0) {
       const int R = run_length();
       if (R > 0) {
@@ -4410,7 +4420,7 @@ __device__ __forceinline__ void prefill_sk2_share(const AttnParams& p,
     }
     // General step.
     const bool seg_start = first || ct == 0;
-    const bool seg_end = ct + 1 == it.T || it.P + kP2ItemCost + ct + 1 >= end;
+    const bool seg_end = ct + 1 == it.T || it.P + kItemCost + ct + 1 >= end;
     first = false;
     step_top(false);
     const int q0 = it.qt * qtile;
@@ -4446,8 +4456,8 @@ __device__ __forceinline__ void prefill_sk2_share(const AttnParams& p,
         plo_dim = dsel;
         plo_keep = L.lm < n_plo ? 0xffffffffu : 0u;
       }
-      const int f = (it.P + kP2ItemCost) / S;
-      const int nseg = (it.P + kP2ItemCost + it.T - 1) / S - f + 1;
+      const int f = (it.P + kItemCost) / S;
+      const int nseg = (it.P + kItemCost + it.T - 1) / S - f + 1;
       split = nseg == 1 ? -1 : w - f;
       nrows = min(qtile, it.geo.sq - q0);
       const int64_t row0 = int64_t(p.n_dec) + it.cq0 + q0;
@@ -4492,13 +4502,13 @@ __device__ __forceinline__ void prefill_sk2_share(const AttnParams& p,
     // out of range).  bf16 rows: lanes lg and lg ^ 1 swap halves first
     // (v_permlane16_swap), so each lane stores 16 contiguous bytes and each
     // row gets 64-byte pieces.
-    const bool next_in = ct + 1 == it.T && it.P + 2 * kP2ItemCost + it.T < end;
+    const bool next_in = ct + 1 == it.T && it.P + 2 * kItemCost + it.T < end;
     if (next_in) {
       // The next item's query into registers (the query registers are dead
       // after this tile's S^T) and the one after into the region, ahead of the
       // stores, so those loads do not queue behind them.
       const PfItem cur = it;
-      p2_next_item(it, ctab, cu_q, cu_k, p.n_pre, kvs_total, p.nslices, qtile);
+      p2_next_item<kItemCost>(it, ctab, cu_q, cu_k, p.n_pre, kvs_total, p.nslices, qtile);
       if (q_for != it.P) {  // defensive: its query is normally issued one item ahead
         issue_q(it);
         q_mark = issued;
@@ -4607,8 +4617,8 @@ __device__ __forceinline__ void prefill_sk2_share(const AttnParams& p,
     }
     if (++ct == it.T) {
       // The next item, if one of its real tiles is in this share.
-      if (it.P + 2 * kP2ItemCost + it.T >= end) break;
-      p2_next_item(it, ctab, cu_q, cu_k, p.n_pre, kvs_total, p.nslices, qtile);
+      if (it.P + 2 * kItemCost + it.T >= end) break;
+      p2_next_item<kItemCost>(it, ctab, cu_q, cu_k, p.n_pre, kvs_total, p.nslices, qtile);
       ct = 0;
     }
   }
