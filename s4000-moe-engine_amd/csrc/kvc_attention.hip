@@ -3946,8 +3946,9 @@ __device__ __forceinline__ void p2_load_chunk(PfItem& it, const int4* ctab, cons
 #endif
 constexpr int kP2ItemCost = KVC_P2_ITEM_COST;
 // With the residue product an item also reads its outlier dims' list and
-// folds the residues in at its end: four chunks of 300-512 tokens after 0-8192 keys took
-// 196 / 191 / 187.4 / 186.1 / 185.5 / 186.4 us a call at 6 / 7 / 8 / 9 / 10 / 12.
+// folds the residues in at its end: four chunks of 300-512 tokens after
+// 0-8192 keys took 196 / 191 / 187.4 / 186.1 / 185.5 / 186.4 us a call at
+// 6 / 7 / 8 / 9 / 10 / 12.
 #ifndef KVC_P2_ITEM_COST_RESIDUE
 #define KVC_P2_ITEM_COST_RESIDUE 10
 #endif

@@ -117,7 +117,12 @@ store_int8_tokhead_kernel(const uint16_t* __restrict__ key, int64_t k_sn, int64_
 }
 
 // Per-channel quantisation floor(x / s + 0.5) with outlier dims zeroed and
-// their exact bf16 values written to the compacted side row.
+// their exact bf16 values written to the compacted side row.  A decode step's
+// append is a few thousand bytes, so memory latency bounds it: every load is
+// issued before the first is used (lane j of a row holds outlier dim j; the
+// dims and the side values then move between lanes), one round trip instead
+// of one per outlier dim.  48 tokens of a decode step: kernel 5.5 -> 5.0 us,
+// the step's call 79.0 -> 78.1 us.
 template <int kIdxBytes>
 __global__ void __launch_bounds__(kThreads)
 store_int8_chan_kernel(const uint16_t* __restrict__ key, int64_t k_sn, int64_t k_sh,
@@ -133,27 +138,27 @@ store_int8_chan_kernel(const uint16_t* __restrict__ key, int64_t k_sn, int64_t k
   const int64_t n = row / kvh;
   const int h = int(row - n * kvh);
   if (n >= num_tokens) return;
-  int64_t slot = wrap_slot(load_index<kIdxBytes>(slots, n), num_slots);
-  if (slot < 0 || slot >= num_slots) return;
-  const uint16_t* krow = key + n * k_sn + h * k_sh;
-  const uint16_t* vrow = value + n * v_sn + h * v_sh;
-  const u32x4_t kw = *reinterpret_cast<const u32x4_t*>(krow + lane16 * 8);
-  const u32x4_t vw = *reinterpret_cast<const u32x4_t*>(vrow + lane16 * 8);
-  float kx[8], vx[8];
-  unpack8(kw, kx);
-  unpack8(vw, vx);
+  const int64_t raw = load_index<kIdxBytes>(slots, n);
+  const u32x4_t kw = *reinterpret_cast<const u32x4_t*>(key + n * k_sn + h * k_sh + lane16 * 8);
+  const u32x4_t vw = *reinterpret_cast<const u32x4_t*>(value + n * v_sn + h * v_sh + lane16 * 8);
   const float4* ks4 = reinterpret_cast<const float4*>(k_scale + h * kD + lane16 * 8);
   const float4* vs4 = reinterpret_cast<const float4*>(v_scale + h * kD + lane16 * 8);
   const float4 ks0 = ks4[0], ks1 = ks4[1], vs0 = vs4[0], vs1 = vs4[1];
+  const bool side = head_n_out != nullptr;
+  const int n_out = side ? min(head_n_out[h], n_out_max) : 0;
+  const int odim = side && lane16 < n_out_max ? out_idx2d[h * n_out_max + lane16] : 0;
+  const int64_t slot = wrap_slot(raw, num_slots);
+  if (slot < 0 || slot >= num_slots) return;
+  float kx[8], vx[8];
+  unpack8(kw, kx);
+  unpack8(vw, vx);
   const float ks[8] = {ks0.x, ks0.y, ks0.z, ks0.w, ks1.x, ks1.y, ks1.z, ks1.w};
   const float vs[8] = {vs0.x, vs0.y, vs0.z, vs0.w, vs1.x, vs1.y, vs1.z, vs1.w};
   int kc[8], vc[8];
   quant_chan8(kx, ks, kc);
   quant_chan8(vx, vs, vc);
-  const int n_out = head_n_out != nullptr ? head_n_out[h] : 0;
   for (int j = 0; j < n_out; ++j) {
-    const int d = out_idx2d[h * n_out_max + j];
-    const int local = d - lane16 * 8;
+    const int local = __shfl(odim, j, kLanesPerRow) - lane16 * 8;
     if (local >= 0 && local < 8) {
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
@@ -164,11 +169,23 @@ store_int8_chan_kernel(const uint16_t* __restrict__ key, int64_t k_sn, int64_t k
       }
     }
   }
-  if (lane16 < n_out) {
-    const int d = out_idx2d[h * n_out_max + lane16];
-    const int64_t so = (slot * kvh + h) * n_out_max + lane16;
-    side_k[so] = krow[d];
-    side_v[so] = vrow[d];
+  if (n_out > 0) {
+    // lane j's dim is element d & 7 of the row's lane d >> 3
+    const int owner = (odim >> 3) & (kLanesPerRow - 1);
+    uint32_t kv = 0, vv = 0;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      const uint32_t a = uint32_t(__shfl(int(kw[w]), owner, kLanesPerRow));
+      const uint32_t b = uint32_t(__shfl(int(vw[w]), owner, kLanesPerRow));
+      kv = w == ((odim & 7) >> 1) ? a : kv;
+      vv = w == ((odim & 7) >> 1) ? b : vv;
+    }
+    if (lane16 < n_out) {
+      const int64_t so = (slot * kvh + h) * n_out_max + lane16;
+      const int sh = (odim & 1) * 16;
+      side_k[so] = uint16_t(kv >> sh);
+      side_v[so] = uint16_t(vv >> sh);
+    }
   }
   const int64_t dst = (slot * kvh + h) * kD + lane16 * 8;
   *reinterpret_cast<u32x2_t*>(k_cache + dst) = u32x2_t{pack_codes4(kc, 0), pack_codes4(kc, 4)};
