@@ -9,6 +9,8 @@ preconditions, RuntimeError for backend failures).
 from __future__ import annotations
 
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 import pathlib
 import threading
@@ -16,6 +18,7 @@ import threading
 import torch
 
 PKG_ROOT = pathlib.Path(__file__).resolve().parent.parent
+HOST_PATH = PKG_ROOT / "lib" / "_kvc_host.so"
 LIB_PATH = pathlib.Path(os.environ.get("KVC_LIBRARY", PKG_ROOT / "lib" / "libkvc.so"))
 
 KVC_KV_BF16 = 0
@@ -127,6 +130,30 @@ def load() -> ctypes.CDLL:
                 _fns[name] = fn
             _lib = lib
     return _lib
+
+
+_host = None
+
+
+def host():
+    """The native host path of the decode step (csrc/kvc_host.cpp), loaded
+    once and bound to libkvc; RuntimeError when it is absent."""
+    global _host
+    if _host is None:
+        load()
+        with _lock:
+            if _host is None:
+                if not HOST_PATH.is_file():
+                    raise RuntimeError(f"_kvc_host.so not found at {HOST_PATH}; build it with "
+                                       f"`make -C {PKG_ROOT / 'csrc'}`")
+                loader = importlib.machinery.ExtensionFileLoader("_kvc_host", str(HOST_PATH))
+                spec = importlib.util.spec_from_file_location("_kvc_host", str(HOST_PATH),
+                                                              loader=loader)
+                module = importlib.util.module_from_spec(spec)
+                loader.exec_module(module)
+                module.bind(str(LIB_PATH))
+                _host = module
+    return _host
 
 
 def call(name: str, *args) -> int:

@@ -55,6 +55,11 @@ def paged_decode_attention(
     k_scale=None, v_scale=None, side_k=None, side_v=None,
     out_idx2d=None, head_n_out=None,
 ):
+    if q.is_cuda and k_scale is None:
+        done = nat.host().decode(None, q, k_cache, v_cache, block_tables, context_lens, scale,
+                                 nat.stream_of(q), None, None, None)
+        if done is not None:
+            return done
     if q.ndim != 3 or k_cache.ndim != 4 or v_cache.shape != k_cache.shape:
         raise ValueError("expected q=[batch,heads,dim], kv=[pages,page,kv_heads,dim]")
     batch, num_heads, head_dim = q.shape
@@ -166,6 +171,11 @@ def decode_append_into(output, q, key, value, k_cache, v_cache, slot_mapping, bl
                        context_lens, scale):
     """paged_decode_append with the result written to `output` ([batch, heads,
     128] bf16, unit inner stride; None: a new tensor), which is returned."""
+    if q.is_cuda:
+        done = nat.host().decode(output, q, k_cache, v_cache, block_tables, context_lens, scale,
+                                 nat.stream_of(q), key, value, slot_mapping)
+        if done is not None:
+            return done
     if q.ndim != 3 or key.ndim != 3 or value.shape != key.shape or k_cache.ndim != 4 \
             or v_cache.shape != k_cache.shape:
         raise ValueError("expected q=[batch,heads,dim], key/value=[batch,kv_heads,dim], "

@@ -48,6 +48,11 @@ def qk_norm_rope_store(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor | None,
     (q_rot, k_rot) with k_rot None when return_k is False.  With k_cache /
     v_cache / slot_mapping the rotated k and the unchanged v are also
     appended to the pool (the engine's store_kvcache semantics)."""
+    if q_out is None and q.is_cuda:
+        done = nat.host().rope(q, k, v, positions, cos_sin_cache, q_norm_weight, k_norm_weight,
+                               eps, k_cache, v_cache, slot_mapping, return_k, nat.stream_of(q))
+        if done is not None:
+            return done
     N, H, D = q.shape
     KVH = k.size(1)
     if D != 128:
