@@ -37,12 +37,33 @@ struct MoveArgs {
   int64_t dst_plane, dst_item;
 };
 
-// One 16 KiB piece of row (item, plane).
+// Block ids passed by value with the launch: a list that the host holds needs
+// no upload (two copies of 4.6 us each ahead of the move, as long as moving a
+// 24 MiB block takes; 16 blocks: 149 -> 141 us a call).
+constexpr int kInlineIds = 256;
+struct InlineIds {
+  int32_t src[kInlineIds];
+  int32_t dst[kInlineIds];
+};
+struct DeviceIds {};
+
+// The blocks item `item` moves from and to (the item itself where no list is
+// given).
+__device__ __forceinline__ void select_blocks(const MoveArgs& a, const DeviceIds&, int64_t item,
+                                              int64_t& s, int64_t& d) {
+  s = a.src_ids ? int64_t(a.src_ids[item]) : item;
+  d = a.dst_ids ? int64_t(a.dst_ids[item]) : item;
+}
+__device__ __forceinline__ void select_blocks(const MoveArgs& a, const InlineIds& ids,
+                                              int64_t item, int64_t& s, int64_t& d) {
+  s = a.src_ids ? int64_t(ids.src[item]) : item;
+  d = a.dst_ids ? int64_t(ids.dst[item]) : item;
+}
+
+// One 16 KiB piece of one row (item, plane).
 template <bool kStream>
-__device__ __forceinline__ void move_piece(const MoveArgs& a, int64_t item, int64_t plane,
-                                           int64_t piece) {
-  const int64_t s_sel = a.src_ids ? int64_t(a.src_ids[item]) : item;
-  const int64_t d_sel = a.dst_ids ? int64_t(a.dst_ids[item]) : item;
+__device__ __forceinline__ void move_piece(const MoveArgs& a, int64_t s_sel, int64_t d_sel,
+                                           int64_t plane, int64_t piece) {
   const char* s = a.src + plane * a.src_plane + s_sel * a.src_item + piece * kPiece;
   char* d = a.dst + plane * a.dst_plane + d_sel * a.dst_item + piece * kPiece;
   const int64_t limit = a.block_bytes - piece * kPiece;
@@ -75,24 +96,30 @@ __device__ __forceinline__ void move_piece(const MoveArgs& a, int64_t item, int6
 // order and plain accesses, 147 us with the XCD order alone, 145 us with
 // non-temporal accesses alone, 134 us (6.0 TB/s) with both; 32 KiB pieces
 // and 1024-thread workgroups 134-137 us; persistent grids 149-160 us (copies
-// alone; the whole BlockMover.copy call, its id uploads included, went from
-// 165 to 148-150 us).
+// alone; the whole BlockMover.copy call, then still uploading its ids, went
+// from 165 to 148-150 us).
 // `total` < 2^31, so 32-bit divisions do.
+template <typename Ids>
 __global__ void __launch_bounds__(kThreads)
-move_blocks_kernel(MoveArgs a, uint32_t total, uint32_t per) {
+move_blocks_kernel(MoveArgs a, uint32_t total, uint32_t per, Ids ids) {
   const uint32_t w = (blockIdx.x & 7u) * per + (blockIdx.x >> 3);
   if ((blockIdx.x >> 3) >= per || w >= total) return;
   const uint32_t row = w / uint32_t(a.pieces);
   const uint32_t item = row / uint32_t(a.planes);
-  move_piece<true>(a, item, row - item * uint32_t(a.planes), w - row * uint32_t(a.pieces));
+  int64_t s, d;
+  select_blocks(a, ids, item, s, d);
+  move_piece<true>(a, s, d, row - item * uint32_t(a.planes), w - row * uint32_t(a.pieces));
 }
 
 // Moves to or from pinned host memory.
-__global__ void __launch_bounds__(kThreads) move_host_kernel(MoveArgs a, int64_t total) {
+template <typename Ids>
+__global__ void __launch_bounds__(kThreads) move_host_kernel(MoveArgs a, int64_t total, Ids ids) {
   for (int64_t w = blockIdx.x; w < total; w += gridDim.x) {
     const int64_t row = w / a.pieces;
     const int64_t item = row / a.planes;
-    move_piece<false>(a, item, row - item * a.planes, w - row * a.pieces);
+    int64_t s, d;
+    select_blocks(a, ids, item, s, d);
+    move_piece<false>(a, s, d, row - item * a.planes, w - row * a.pieces);
   }
 }
 
@@ -105,22 +132,48 @@ int64_t host_move_workgroups() {
   return wgs;
 }
 
-int launch_move(const MoveArgs& a, int64_t n, hipStream_t st, const char* what,
-                bool host_side = false) {
-  if (n == 0 || a.planes == 0 || a.block_bytes == 0) return KVC_OK;
+template <typename Ids>
+int launch_one(const MoveArgs& a, int64_t n, hipStream_t st, const char* what, bool host_side,
+               const Ids& ids) {
   const int64_t total = n * a.planes * a.pieces;
   if (host_side) {
     const int64_t grid = std::min(total, host_move_workgroups());
     KVC_REQUIRE(grid < (int64_t(1) << 31), KVC_ERR_VALUE, "%s: %lld workgroups exceed one launch",
                 what, (long long)grid);
-    move_host_kernel<<<unsigned(grid), kThreads, 0, st>>>(a, total);
+    move_host_kernel<<<unsigned(grid), kThreads, 0, st>>>(a, total, ids);
     return check_launch(what);
   }
   KVC_REQUIRE(total < (int64_t(1) << 31), KVC_ERR_VALUE, "%s: %lld workgroups exceed one launch",
               what, (long long)total);
   const uint32_t per = uint32_t((total + 7) / 8);
-  move_blocks_kernel<<<8 * per, kThreads, 0, st>>>(a, uint32_t(total), per);
+  move_blocks_kernel<<<8 * per, kThreads, 0, st>>>(a, uint32_t(total), per, ids);
   return check_launch(what);
+}
+
+// ids_on_host: a.src_ids / a.dst_ids are host arrays, read before the call
+// returns and passed with the launches, kInlineIds items each.
+int launch_move(const MoveArgs& a, int64_t n, hipStream_t st, const char* what,
+                bool host_side = false, bool ids_on_host = false) {
+  if (n == 0 || a.planes == 0 || a.block_bytes == 0) return KVC_OK;
+  if (!ids_on_host) return launch_one(a, n, st, what, host_side, DeviceIds{});
+  for (int64_t i0 = 0; i0 < n; i0 += kInlineIds) {
+    const int64_t m = std::min<int64_t>(kInlineIds, n - i0);
+    InlineIds ids;
+    MoveArgs part = a;
+    if (a.src_ids != nullptr) {
+      std::copy(a.src_ids + i0, a.src_ids + i0 + m, ids.src);
+    } else {
+      part.src = a.src + i0 * a.src_item;
+    }
+    if (a.dst_ids != nullptr) {
+      std::copy(a.dst_ids + i0, a.dst_ids + i0 + m, ids.dst);
+    } else {
+      part.dst = a.dst + i0 * a.dst_item;
+    }
+    const int rc = launch_one(part, m, st, what, host_side, ids);
+    if (rc != KVC_OK) return rc;
+  }
+  return KVC_OK;
 }
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
@@ -171,10 +224,12 @@ int check_geometry(const void* a, const void* b, int64_t planes, int64_t block_b
 
 using namespace kvc;
 
-extern "C" int kvc_block_gather(const void* src, int64_t planes, int64_t src_plane_stride,
+namespace {
+int block_gather(const void* src, int64_t planes, int64_t src_plane_stride,
                                 int64_t block_bytes, const int32_t* block_ids, int64_t n,
                                 void* dst, int64_t dst_item_stride, int64_t dst_plane_stride,
-                                kvc_stream_t stream) {
+                                kvc_stream_t stream,
+    bool ids_on_host) {
   clear_error();
   int rc = check_geometry(src, dst, planes, block_bytes,
                           {src_plane_stride, dst_item_stride, dst_plane_stride}, n,
@@ -197,13 +252,29 @@ extern "C" int kvc_block_gather(const void* src, int64_t planes, int64_t src_pla
   a.dst_ids = nullptr;
   a.dst_plane = dst_plane_stride;
   a.dst_item = dst_item_stride;
-  return launch_move(a, n, as_stream(stream), "block_gather", host_side);
+  return launch_move(a, n, as_stream(stream), "block_gather", host_side, ids_on_host);
+}
+}  // namespace
+
+extern "C" int kvc_block_gather(const void* src, int64_t planes, int64_t src_plane_stride,
+                                int64_t block_bytes, const int32_t* block_ids, int64_t n,
+                                void* dst, int64_t dst_item_stride, int64_t dst_plane_stride,
+                                kvc_stream_t stream) {
+  return block_gather(src, planes, src_plane_stride, block_bytes, block_ids, n, dst, dst_item_stride, dst_plane_stride, stream, false);
+}
+extern "C" int kvc_block_gather_ids(const void* src, int64_t planes, int64_t src_plane_stride,
+                                int64_t block_bytes, const int32_t* block_ids, int64_t n,
+                                void* dst, int64_t dst_item_stride, int64_t dst_plane_stride,
+                                kvc_stream_t stream) {
+  return block_gather(src, planes, src_plane_stride, block_bytes, block_ids, n, dst, dst_item_stride, dst_plane_stride, stream, true);
 }
 
-extern "C" int kvc_block_scatter(const void* src, int64_t src_item_stride,
+namespace {
+int block_scatter(const void* src, int64_t src_item_stride,
                                  int64_t src_plane_stride, int64_t planes, int64_t block_bytes,
                                  const int32_t* block_ids, int64_t n, void* dst,
-                                 int64_t dst_plane_stride, kvc_stream_t stream) {
+                                 int64_t dst_plane_stride, kvc_stream_t stream,
+    bool ids_on_host) {
   clear_error();
   int rc = check_geometry(src, dst, planes, block_bytes,
                           {src_item_stride, src_plane_stride, dst_plane_stride}, n,
@@ -226,12 +297,28 @@ extern "C" int kvc_block_scatter(const void* src, int64_t src_item_stride,
   a.dst_ids = block_ids;
   a.dst_plane = dst_plane_stride;
   a.dst_item = block_bytes;
-  return launch_move(a, n, as_stream(stream), "block_scatter", host_side);
+  return launch_move(a, n, as_stream(stream), "block_scatter", host_side, ids_on_host);
+}
+}  // namespace
+
+extern "C" int kvc_block_scatter(const void* src, int64_t src_item_stride,
+                                 int64_t src_plane_stride, int64_t planes, int64_t block_bytes,
+                                 const int32_t* block_ids, int64_t n, void* dst,
+                                 int64_t dst_plane_stride, kvc_stream_t stream) {
+  return block_scatter(src, src_item_stride, src_plane_stride, planes, block_bytes, block_ids, n, dst, dst_plane_stride, stream, false);
+}
+extern "C" int kvc_block_scatter_ids(const void* src, int64_t src_item_stride,
+                                 int64_t src_plane_stride, int64_t planes, int64_t block_bytes,
+                                 const int32_t* block_ids, int64_t n, void* dst,
+                                 int64_t dst_plane_stride, kvc_stream_t stream) {
+  return block_scatter(src, src_item_stride, src_plane_stride, planes, block_bytes, block_ids, n, dst, dst_plane_stride, stream, true);
 }
 
-extern "C" int kvc_block_copy(void* pool, int64_t planes, int64_t plane_stride,
+namespace {
+int block_copy(void* pool, int64_t planes, int64_t plane_stride,
                               int64_t block_bytes, const int32_t* src_ids, const int32_t* dst_ids,
-                              int64_t n, kvc_stream_t stream) {
+                              int64_t n, kvc_stream_t stream,
+    bool ids_on_host) {
   clear_error();
   int rc = check_geometry(pool, pool, planes, block_bytes, {plane_stride}, n, "block_copy");
   if (rc != KVC_OK) return rc;
@@ -249,7 +336,19 @@ extern "C" int kvc_block_copy(void* pool, int64_t planes, int64_t plane_stride,
   a.dst_ids = dst_ids;
   a.dst_plane = plane_stride;
   a.dst_item = block_bytes;
-  return launch_move(a, n, as_stream(stream), "block_copy");
+  return launch_move(a, n, as_stream(stream), "block_copy", false, ids_on_host);
+}
+}  // namespace
+
+extern "C" int kvc_block_copy(void* pool, int64_t planes, int64_t plane_stride,
+                              int64_t block_bytes, const int32_t* src_ids, const int32_t* dst_ids,
+                              int64_t n, kvc_stream_t stream) {
+  return block_copy(pool, planes, plane_stride, block_bytes, src_ids, dst_ids, n, stream, false);
+}
+extern "C" int kvc_block_copy_ids(void* pool, int64_t planes, int64_t plane_stride,
+                              int64_t block_bytes, const int32_t* src_ids, const int32_t* dst_ids,
+                              int64_t n, kvc_stream_t stream) {
+  return block_copy(pool, planes, plane_stride, block_bytes, src_ids, dst_ids, n, stream, true);
 }
 
 extern "C" int kvc_block_d2h(const void* pool, int64_t planes, int64_t plane_stride,

@@ -93,8 +93,11 @@ SIGNATURES = {
     "kvc_gather_kv": (_INT, [_P, _P, _I64, _I64, _I64, _I64, _INT, _P, _P, _P, _P, _P, _P,
                              _I64, _P, _I64, _I64, _I64, _I64, _P, _I64, _P, _P, _P]),
     "kvc_block_gather": (_INT, [_P, _I64, _I64, _I64, _P, _I64, _P, _I64, _I64, _P]),
+    "kvc_block_gather_ids": (_INT, [_P, _I64, _I64, _I64, _P, _I64, _P, _I64, _I64, _P]),
     "kvc_block_scatter": (_INT, [_P, _I64, _I64, _I64, _I64, _P, _I64, _P, _I64, _P]),
+    "kvc_block_scatter_ids": (_INT, [_P, _I64, _I64, _I64, _I64, _P, _I64, _P, _I64, _P]),
     "kvc_block_copy": (_INT, [_P, _I64, _I64, _I64, _P, _P, _I64, _P]),
+    "kvc_block_copy_ids": (_INT, [_P, _I64, _I64, _I64, _P, _P, _I64, _P]),
     "kvc_block_d2h": (_INT, [_P, _I64, _I64, _I64, _P, _I64, _P, _I64, _P]),
     "kvc_block_h2d": (_INT, [_P, _I64, _I64, _I64, _P, _I64, _P, _I64, _P]),
     "kvc_qk_norm_rope_store": (_INT, [_P, _I64, _I64, _P, _I64, _I64, _P, _I64, _I64,

@@ -47,12 +47,16 @@ class BlockMover:
         self.item_bytes = self.planes * self.block_bytes
 
     # -- helpers ---------------------------------------------------------
-    def _dev_ids(self, ids) -> torch.Tensor:
-        if isinstance(ids, torch.Tensor):
+    def _ids(self, ids) -> tuple[torch.Tensor, str]:
+        """int32 block ids where they are, and the entry-point suffix: a
+        device tensor stays on the device; a list (or a host tensor) goes
+        with the launch, without an upload."""
+        if isinstance(ids, torch.Tensor) and ids.is_cuda:
             t = ids.to(device=self.pool.device, dtype=torch.int32)
-        else:
-            t = torch.as_tensor(list(ids), dtype=torch.int32).to(self.pool.device, non_blocking=True)
-        return t.contiguous()
+            return t.contiguous(), ""
+        if not isinstance(ids, torch.Tensor):
+            ids = torch.as_tensor(list(ids), dtype=torch.int32)
+        return ids.to(dtype=torch.int32).contiguous(), "_ids"
 
     def _host_ids(self, ids) -> np.ndarray:
         if isinstance(ids, torch.Tensor):
@@ -82,9 +86,9 @@ class BlockMover:
         self._check_items(out, n)
         if n == 0:
             return out
-        dev_ids = self._dev_ids(ids)
-        nat.call("kvc_block_gather", self.pool.data_ptr(), self.planes, self.plane_stride,
-                 self.block_bytes, dev_ids.data_ptr(), n, out.data_ptr(), self.item_bytes,
+        t, form = self._ids(ids)
+        nat.call("kvc_block_gather" + form, self.pool.data_ptr(), self.planes, self.plane_stride,
+                 self.block_bytes, t.data_ptr(), n, out.data_ptr(), self.item_bytes,
                  self.block_bytes, self._stream())
         return out
 
@@ -94,9 +98,9 @@ class BlockMover:
         self._check_items(items, n)
         if n == 0:
             return
-        dev_ids = self._dev_ids(ids)
-        nat.call("kvc_block_scatter", items.data_ptr(), self.item_bytes, self.block_bytes,
-                 self.planes, self.block_bytes, dev_ids.data_ptr(), n, self.pool.data_ptr(),
+        t, form = self._ids(ids)
+        nat.call("kvc_block_scatter" + form, items.data_ptr(), self.item_bytes, self.block_bytes,
+                 self.planes, self.block_bytes, t.data_ptr(), n, self.pool.data_ptr(),
                  self.plane_stride, self._stream())
 
     def copy(self, src_ids, dst_ids) -> None:
@@ -114,8 +118,8 @@ class BlockMover:
             staged = self.gather(src)
             self.scatter(staged, dst)
             return
-        s, d = self._dev_ids(src), self._dev_ids(dst)
-        nat.call("kvc_block_copy", self.pool.data_ptr(), self.planes, self.plane_stride,
+        (s, form), (d, _) = self._ids(src), self._ids(dst)
+        nat.call("kvc_block_copy" + form, self.pool.data_ptr(), self.planes, self.plane_stride,
                  self.block_bytes, s.data_ptr(), d.data_ptr(), len(src), self._stream())
 
     # -- copy engines ----------------------------------------------------

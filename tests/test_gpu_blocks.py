@@ -118,6 +118,7 @@ def test_overlapped_swap_step_matches_sequential_moves():
     (1, 16 * 1024, 7),             # one full piece per row, 7 pieces over 8 XCDs
     (3, 16 * 1024 + 16, 3),        # a second piece of one vector; 18 pieces
     (5, 3 * 16 * 1024 - 16, 13),   # a last piece one vector short; 195 pieces
+    (2, 48, 256), (2, 48, 257), (1, 16, 600),  # 256 host ids go with one launch
 ])
 def test_device_moves_at_piece_and_xcd_edges(planes, row_bytes, n):
     g = torch.Generator().manual_seed(7)
@@ -130,10 +131,19 @@ def test_device_moves_at_piece_and_xcd_edges(planes, row_bytes, n):
     print(f"[blocks] edges planes={planes} row={row_bytes} n={n}", flush=True)
     items = mover.gather(src)
     assert torch.equal(items, before[:, :, src].movedim(2, 0))
+    # ids on the device (read there) and in a pinned-host destination's move
+    assert torch.equal(mover.gather(torch.tensor(src, device=DEV)), items)
+    host = torch.empty_like(items, device="cpu", pin_memory=True)
+    mover.gather(torch.tensor(src), out=host)
+    torch.cuda.synchronize()
+    assert torch.equal(host, items.cpu())
     expect = before.clone()
     expect[:, :, dst] = before[:, :, src]
     mover.copy(src, dst)
     assert torch.equal(pool, expect)
     expect[:, :, src] = items.movedim(0, 2).flip(2)
     mover.scatter(items.flip(0), src)
+    assert torch.equal(pool, expect)
+    expect[:, :, src] = items.movedim(0, 2)
+    mover.scatter(host, src)
     assert torch.equal(pool, expect)
