@@ -8,7 +8,7 @@
 // and returns None, having done nothing, for anything else: the Python
 // function then checks, converts or raises as it always did.  Nothing is
 // kept between calls.  Measured: one row of 333 tokens through norm, rotary,
-// append and attention (16 q / 8 kv heads) 30.1 -> 18.4 us a pass, a decode
+// append and attention (16 q / 8 kv heads) 30 -> 16-18 us a pass, a decode
 // step of 11 rows of 97-1501 tokens 20.0 -> 14.7 us (both now GPU-bound).
 #include <Python.h>
 

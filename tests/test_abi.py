@@ -229,3 +229,15 @@ def test_mixed_split_from_the_work_hints(monkeypatch):
     assert split(60, cfg3) == 64
     monkeypatch.setenv("KVC_MIXED_DECODE_CUS", "0")
     assert split(60, cfg3) == 0
+
+
+def test_host_extension_has_no_thread_local_storage():
+    # A TLS segment in a library loaded after startup slows every later TLS
+    # access of the process (see the Makefile).
+    import struct
+    data = _native.HOST_PATH.read_bytes()
+    assert data[:6] == b"\x7fELF\x02\x01"
+    phoff, = struct.unpack_from("<Q", data, 32)
+    size, count = struct.unpack_from("<HH", data, 54)
+    types = [struct.unpack_from("<I", data, phoff + i * size)[0] for i in range(count)]
+    assert 1 in types and 7 not in types  # PT_LOAD, no PT_TLS
