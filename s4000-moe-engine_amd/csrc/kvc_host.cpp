@@ -81,6 +81,14 @@ PyObject* fail(int rc, const char* what) {
   return nullptr;
 }
 
+// A torch C++ exception (an allocation that fails, a tensor without storage):
+// nothing has been launched, so the Python path takes the call and raises its
+// own error (torch.OutOfMemoryError, not a plain RuntimeError).
+PyObject* declined() {
+  PyErr_Clear();
+  Py_RETURN_NONE;
+}
+
 // decode(out or None, q, k_cache, v_cache, block_tables, context_lens, scale,
 //        stream, key or None, value, slot_mapping)
 PyObject* decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
@@ -152,9 +160,8 @@ PyObject* decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
       return a[0];
     }
     return THPVariable_Wrap(std::move(out));
-  } catch (const std::exception& e) {
-    PyErr_SetString(PyExc_RuntimeError, e.what());
-    return nullptr;
+  } catch (const std::exception&) {
+    return declined();
   }
 }
 
@@ -234,9 +241,8 @@ PyObject* rope(PyObject*, PyObject* const* a, Py_ssize_t n) {
       PyTuple_SET_ITEM(r, 1, Py_None);
     }
     return r;
-  } catch (const std::exception& e) {
-    PyErr_SetString(PyExc_RuntimeError, e.what());
-    return nullptr;
+  } catch (const std::exception&) {
+    return declined();
   }
 }
 
