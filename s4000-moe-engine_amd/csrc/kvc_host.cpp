@@ -81,12 +81,43 @@ PyObject* fail(int rc, const char* what) {
   return nullptr;
 }
 
-// A torch C++ exception (an allocation that fails, a tensor without storage):
-// nothing has been launched, so the Python path takes the call and raises its
-// own error (torch.OutOfMemoryError, not a plain RuntimeError).
+// A torch C++ exception before the launch (an allocation that fails, a tensor
+// without storage): the Python path takes the call and raises its own error
+// (torch.OutOfMemoryError, not a plain RuntimeError).
 PyObject* declined() {
   PyErr_Clear();
   Py_RETURN_NONE;
+}
+
+// Every torch call that can throw (data_ptr() of a tensor without storage
+// among them) comes before a launch, with the interpreter lock held; Unlocked
+// covers the library call alone.
+struct Unlocked {
+  PyThreadState* state = PyEval_SaveThread();
+  Unlocked() = default;
+  Unlocked(const Unlocked&) = delete;
+  ~Unlocked() { PyEval_RestoreThread(state); }
+};
+
+// A tensor of a call as the library takes it.
+struct Rows {
+  void* p = nullptr;
+  int64_t s0 = 0, s1 = 0;
+};
+Rows rows(const at::Tensor* t) {
+  return t != nullptr && t->defined() ? Rows{t->data_ptr(), t->stride(0), t->stride(1)} : Rows{};
+}
+void* address(const at::Tensor* t) { return t != nullptr ? t->data_ptr() : nullptr; }
+
+// A new reference to `t` after a launch: an error here is raised, the call is
+// not made again.
+PyObject* wrap(at::Tensor&& t) {
+  try {
+    return THPVariable_Wrap(std::move(t));
+  } catch (const std::exception& e) {
+    if (!PyErr_Occurred()) PyErr_SetString(PyExc_RuntimeError, e.what());
+    return nullptr;
+  }
 }
 
 // decode(out or None, q, k_cache, v_cache, block_tables, context_lens, scale,
@@ -96,16 +127,23 @@ PyObject* decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
     PyErr_SetString(PyExc_TypeError, "decode takes 11 arguments");
     return nullptr;
   }
+  at::Tensor out, ws;
+  Rows q_r, k_r, v_r, out_r;
+  void *slots_p, *kc_p, *vc_p, *bt_p, *lens_p, *ws_p, *stream;
+  int64_t batch, heads, kvh, pages, page, bt_stride, blocks;
+  size_t bytes;
+  float scale;
+  int sb = 4;
+  const bool append = a[8] != Py_None;
   try {
     const at::Tensor* q = tensor(a[1]);
     if (q == nullptr || !q->defined() || !plain(q, at::kBFloat16, 3, *q)) Py_RETURN_NONE;
     const at::Tensor *kc = tensor(a[2]), *vc = tensor(a[3]), *bt = tensor(a[4]),
                      *lens = tensor(a[5]);
     if (!decode_shapes(*q, kc, vc, bt, lens) || !PyFloat_CheckExact(a[6])) Py_RETURN_NONE;
-    const int64_t batch = q->size(0), heads = q->size(1), kvh = kc->size(2);
-    const bool append = a[8] != Py_None;
+    batch = q->size(0), heads = q->size(1), kvh = kc->size(2);
+    pages = kc->size(0), page = kc->size(1), bt_stride = bt->stride(0), blocks = bt->size(1);
     const at::Tensor *key = nullptr, *value = nullptr, *slots = nullptr;
-    int sb = 4;
     if (append) {
       key = tensor(a[8]);
       value = tensor(a[9]);
@@ -117,7 +155,6 @@ PyObject* decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
           !is_index(slots, batch, *q, &sb) || (check != nullptr && std::strcmp(check, "1") == 0))
         Py_RETURN_NONE;
     }
-    at::Tensor out;
     if (a[0] != Py_None) {
       const at::Tensor* given = tensor(a[0]);
       if (!plain(given, at::kBFloat16, 3, *q) || given->sizes() != q->sizes() ||
@@ -127,42 +164,40 @@ PyObject* decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
     } else {
       out = output_like(*q);
     }
-    void* stream = PyLong_AsVoidPtr(a[7]);
+    stream = PyLong_AsVoidPtr(a[7]);
     if (PyErr_Occurred()) return nullptr;
-    const float scale = float(PyFloat_AS_DOUBLE(a[6]));
-    const size_t bytes = p_workspace(batch, heads, kvh, 128, kc->size(1), bt->size(1));
-    at::Tensor ws;
+    scale = float(PyFloat_AS_DOUBLE(a[6]));
+    bytes = p_workspace(batch, heads, kvh, 128, page, blocks);
     if (bytes > 0) ws = at::empty({int64_t(bytes)}, q->options().dtype(at::kByte));
-    void* wp = bytes > 0 ? ws.data_ptr() : nullptr;
-    int rc;
-    Py_BEGIN_ALLOW_THREADS;
-    if (append) {
-      rc = p_decode_append(q->data_ptr(), q->stride(0), q->stride(1), key->data_ptr(),
-                           key->stride(0), key->stride(1), value->data_ptr(), value->stride(0),
-                           value->stride(1), slots->data_ptr(), sb, kc->data_ptr(),
-                           vc->data_ptr(), kc->size(0), kc->size(1), kvh, 128,
-                           static_cast<const int32_t*>(bt->data_ptr()), bt->stride(0),
-                           bt->size(1), static_cast<const int32_t*>(lens->data_ptr()), batch,
-                           heads, scale, out.data_ptr(), out.stride(0), out.stride(1), wp, bytes,
-                           stream);
-    } else {
-      rc = p_decode(q->data_ptr(), q->stride(0), q->stride(1), kc->data_ptr(), vc->data_ptr(),
-                    kc->size(0), kc->size(1), kvh, 128, KVC_KV_BF16, nullptr, nullptr, nullptr,
-                    nullptr, nullptr, nullptr, 0, static_cast<const int32_t*>(bt->data_ptr()),
-                    bt->stride(0), bt->size(1), static_cast<const int32_t*>(lens->data_ptr()),
-                    batch, heads, scale, out.data_ptr(), out.stride(0), out.stride(1), wp, bytes,
-                    stream);
-    }
-    Py_END_ALLOW_THREADS;
-    if (rc != KVC_OK) return fail(rc, "paged_decode");
-    if (a[0] != Py_None) {
-      Py_INCREF(a[0]);
-      return a[0];
-    }
-    return THPVariable_Wrap(std::move(out));
+    ws_p = bytes > 0 ? ws.data_ptr() : nullptr;
+    q_r = rows(q), k_r = rows(key), v_r = rows(value), out_r = rows(&out);
+    slots_p = address(slots);
+    kc_p = address(kc), vc_p = address(vc), bt_p = address(bt), lens_p = address(lens);
   } catch (const std::exception&) {
     return declined();
   }
+  int rc;
+  if (append) {
+    Unlocked unlocked;
+    rc = p_decode_append(q_r.p, q_r.s0, q_r.s1, k_r.p, k_r.s0, k_r.s1, v_r.p, v_r.s0, v_r.s1,
+                         slots_p, sb, kc_p, vc_p, pages, page, kvh, 128,
+                         static_cast<const int32_t*>(bt_p), bt_stride, blocks,
+                         static_cast<const int32_t*>(lens_p), batch, heads, scale, out_r.p,
+                         out_r.s0, out_r.s1, ws_p, bytes, stream);
+  } else {
+    Unlocked unlocked;
+    rc = p_decode(q_r.p, q_r.s0, q_r.s1, kc_p, vc_p, pages, page, kvh, 128, KVC_KV_BF16, nullptr,
+                  nullptr, nullptr, nullptr, nullptr, nullptr, 0,
+                  static_cast<const int32_t*>(bt_p), bt_stride, blocks,
+                  static_cast<const int32_t*>(lens_p), batch, heads, scale, out_r.p, out_r.s0,
+                  out_r.s1, ws_p, bytes, stream);
+  }
+  if (rc != KVC_OK) return fail(rc, "paged_decode");
+  if (a[0] != Py_None) {
+    Py_INCREF(a[0]);
+    return a[0];
+  }
+  return wrap(std::move(out));
 }
 
 // rope(q, k, v or None, positions, cos_sin, q_weight or None, k_weight or
@@ -172,14 +207,19 @@ PyObject* rope(PyObject*, PyObject* const* a, Py_ssize_t n) {
     PyErr_SetString(PyExc_TypeError, "rope takes 13 arguments");
     return nullptr;
   }
+  at::Tensor q_out, k_out;
+  Rows q_r, k_r, v_r, qo_r, ko_r;
+  void *pos_p, *cs_p, *qw_p, *kw_p, *kc_p, *vc_p, *slots_p, *stream;
+  int64_t tokens, heads, kvh, max_position, num_slots = 0;
+  int pb = 4, sb = 4;
+  float eps;
   try {
     const at::Tensor *q = tensor(a[0]), *k = tensor(a[1]), *pos = tensor(a[3]),
                      *cs = tensor(a[4]);
     if (q == nullptr || !q->defined() || !plain(q, at::kBFloat16, 3, *q) ||
         !plain(k, at::kBFloat16, 3, *q) || !plain(cs, at::kFloat, 2, *q))
       Py_RETURN_NONE;
-    const int64_t tokens = q->size(0), heads = q->size(1), kvh = k->size(1);
-    int pb = 4, sb = 4;
+    tokens = q->size(0), heads = q->size(1), kvh = k->size(1);
     if (tokens == 0 || q->size(2) != 128 || k->size(0) != tokens || k->size(2) != 128 ||
         kvh == 0 || heads == 0 || q->stride(2) != 1 || k->stride(2) != 1 || cs->size(1) != 128 ||
         !cs->is_contiguous() || !is_index(pos, tokens, *q, &pb) || !PyFloat_CheckExact(a[7]) ||
@@ -198,9 +238,8 @@ PyObject* rope(PyObject*, PyObject* const* a, Py_ssize_t n) {
       if (!plain(v, at::kBFloat16, 3, *q) || v->sizes() != k->sizes() || v->stride(2) != 1)
         Py_RETURN_NONE;
     }
-    const bool cache = a[8] != Py_None;
     const at::Tensor *kc = nullptr, *vc = nullptr, *slots = nullptr;
-    if (cache) {
+    if (a[8] != Py_None) {
       kc = tensor(a[8]);
       vc = tensor(a[9]);
       slots = tensor(a[10]);
@@ -208,42 +247,44 @@ PyObject* rope(PyObject*, PyObject* const* a, Py_ssize_t n) {
           kc->sizes() != vc->sizes() || !kc->is_contiguous() || !vc->is_contiguous() ||
           !is_index(slots, tokens, *q, &sb))
         Py_RETURN_NONE;
+      num_slots = kc->numel() / (kvh * 128);
     }
-    void* stream = PyLong_AsVoidPtr(a[12]);
+    stream = PyLong_AsVoidPtr(a[12]);
     if (PyErr_Occurred()) return nullptr;
-    const float eps = float(PyFloat_AS_DOUBLE(a[7]));
-    at::Tensor q_out = at::empty({tokens, heads, 128}, q->options());
-    at::Tensor k_out;
+    eps = float(PyFloat_AS_DOUBLE(a[7]));
+    max_position = cs->size(0);
+    q_out = at::empty({tokens, heads, 128}, q->options());
     if (a[11] == Py_True) k_out = at::empty({tokens, kvh, 128}, k->options());
-    const bool ko = k_out.defined();
-    int rc;
-    Py_BEGIN_ALLOW_THREADS;
-    rc = p_rope(q->data_ptr(), q->stride(0), q->stride(1), k->data_ptr(), k->stride(0),
-                k->stride(1), v != nullptr ? v->data_ptr() : nullptr,
-                v != nullptr ? v->stride(0) : 0, v != nullptr ? v->stride(1) : 0, tokens, heads,
-                kvh, 128, pos->data_ptr(), pb, w[0] != nullptr ? w[0]->data_ptr() : nullptr,
-                w[1] != nullptr ? w[1]->data_ptr() : nullptr, eps,
-                static_cast<const float*>(cs->data_ptr()), cs->size(0), q_out.data_ptr(),
-                q_out.stride(0), q_out.stride(1), ko ? k_out.data_ptr() : nullptr,
-                ko ? k_out.stride(0) : 0, ko ? k_out.stride(1) : 0,
-                cache ? kc->data_ptr() : nullptr, cache ? vc->data_ptr() : nullptr,
-                cache ? kc->numel() / (kvh * 128) : 0, cache ? slots->data_ptr() : nullptr, sb,
-                stream);
-    Py_END_ALLOW_THREADS;
-    if (rc != KVC_OK) return fail(rc, "kvc_qk_norm_rope_store");
-    PyObject* r = PyTuple_New(2);
-    if (r == nullptr) return nullptr;
-    PyTuple_SET_ITEM(r, 0, THPVariable_Wrap(std::move(q_out)));
-    if (ko) {
-      PyTuple_SET_ITEM(r, 1, THPVariable_Wrap(std::move(k_out)));
-    } else {
-      Py_INCREF(Py_None);
-      PyTuple_SET_ITEM(r, 1, Py_None);
-    }
-    return r;
+    q_r = rows(q), k_r = rows(k), v_r = rows(v), qo_r = rows(&q_out), ko_r = rows(&k_out);
+    pos_p = address(pos), cs_p = address(cs), qw_p = address(w[0]), kw_p = address(w[1]);
+    kc_p = address(kc), vc_p = address(vc), slots_p = address(slots);
   } catch (const std::exception&) {
     return declined();
   }
+  int rc;
+  {
+    Unlocked unlocked;
+    rc = p_rope(q_r.p, q_r.s0, q_r.s1, k_r.p, k_r.s0, k_r.s1, v_r.p, v_r.s0, v_r.s1, tokens,
+                heads, kvh, 128, pos_p, pb, qw_p, kw_p, eps, static_cast<const float*>(cs_p),
+                max_position, qo_r.p, qo_r.s0, qo_r.s1, ko_r.p, ko_r.s0, ko_r.s1, kc_p, vc_p,
+                num_slots, slots_p, sb, stream);
+  }
+  if (rc != KVC_OK) return fail(rc, "kvc_qk_norm_rope_store");
+  PyObject* r = PyTuple_New(2);
+  if (r == nullptr) return nullptr;
+  PyObject* q_py = wrap(std::move(q_out));
+  PyObject* k_py = nullptr;
+  if (ko_r.p != nullptr) {
+    k_py = wrap(std::move(k_out));
+  } else {
+    Py_INCREF(Py_None);
+    k_py = Py_None;
+  }
+  PyTuple_SET_ITEM(r, 0, q_py);
+  PyTuple_SET_ITEM(r, 1, k_py);
+  if (q_py != nullptr && k_py != nullptr) return r;
+  Py_DECREF(r);
+  return nullptr;
 }
 
 template <typename F>
