@@ -248,6 +248,8 @@ PyObject* rope(PyObject*, PyObject* const* a, Py_ssize_t n) {
           !is_index(slots, tokens, *q, &sb))
         Py_RETURN_NONE;
       num_slots = kc->numel() / (kvh * 128);
+    } else if (a[9] != Py_None) {
+      Py_RETURN_NONE;  // a v pool alone is refused
     }
     stream = PyLong_AsVoidPtr(a[12]);
     if (PyErr_Occurred()) return nullptr;

@@ -194,3 +194,15 @@ def test_rope_forms(monkeypatch, tokens, form, return_k):
     assert isinstance(native[0], type) == (form == "half table")
     assert _same(native[0], python[0])
     assert _same(native[1], python[1])
+
+
+def test_rope_refuses_a_v_pool_alone():
+    q, k, v = (torch.zeros(3, h, 128, dtype=torch.bfloat16, device=DEV) for h in (16, 8, 8))
+    pos = torch.arange(3, device=DEV)
+    cs = build_cos_sin_cache(128, 16, 1e6, DEV)
+    pool = torch.zeros(1, PAGE, 8, 128, dtype=torch.bfloat16, device=DEV)
+    print("[host] rope with a v pool alone", flush=True)
+    with pytest.raises(ValueError, match="both caches"):
+        qk_norm_rope_store(q, k, v, pos, cs, v_cache=pool, slot_mapping=pos.int())
+    with pytest.raises(ValueError, match="v_cache"):
+        qk_norm_rope_store(q, k, v, pos, cs, k_cache=pool, slot_mapping=pos.int())
