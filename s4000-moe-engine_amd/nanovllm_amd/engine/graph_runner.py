@@ -163,20 +163,22 @@ class DecodeGraphRunner:
         """Bucket b's static buffers from a batch of bs rows."""
         if bs > 0 and self.head_dim % 8 == 0 and self.q.element_size() == 2 \
                 and self._stageable(bs, q, k, v, slot_mapping, context_lens, block_tables):
-            nat.call(
-                "kvc_stage_decode",
-                q.data_ptr(), q.stride(0) * 2, q.stride(1) * 2,
-                k.data_ptr(), k.stride(0) * 2, k.stride(1) * 2,
-                v.data_ptr(), v.stride(0) * 2, v.stride(1) * 2,
-                self.num_heads * self.head_dim * 2, self.num_kv_heads * self.head_dim * 2,
-                self.num_layers, bs, b, self.max_bs,
-                slot_mapping.data_ptr(), slot_mapping.element_size(),
-                context_lens.data_ptr(), context_lens.element_size(),
-                block_tables.data_ptr(), block_tables.stride(0), block_tables.size(1),
-                self.q.data_ptr(), self.k.data_ptr(), self.v.data_ptr(),
-                self.slot_mapping.data_ptr(), self.context_lens.data_ptr(),
-                self.block_tables.data_ptr(), self.block_tables.size(1),
-                self.scratch_slot, self.scratch_block_id, nat.stream_of(self.q))
+            # A default stream's handle names the current device's stream.
+            with torch.cuda.device(self.q.device):
+                nat.call(
+                    "kvc_stage_decode",
+                    q.data_ptr(), q.stride(0) * 2, q.stride(1) * 2,
+                    k.data_ptr(), k.stride(0) * 2, k.stride(1) * 2,
+                    v.data_ptr(), v.stride(0) * 2, v.stride(1) * 2,
+                    self.num_heads * self.head_dim * 2, self.num_kv_heads * self.head_dim * 2,
+                    self.num_layers, bs, b, self.max_bs,
+                    slot_mapping.data_ptr(), slot_mapping.element_size(),
+                    context_lens.data_ptr(), context_lens.element_size(),
+                    block_tables.data_ptr(), block_tables.stride(0), block_tables.size(1),
+                    self.q.data_ptr(), self.k.data_ptr(), self.v.data_ptr(),
+                    self.slot_mapping.data_ptr(), self.context_lens.data_ptr(),
+                    self.block_tables.data_ptr(), self.block_tables.size(1),
+                    self.scratch_slot, self.scratch_block_id, nat.stream_of(self.q))
             return
         self.q[:, :bs] = q
         self.k[:, :bs] = k

@@ -2,9 +2,13 @@
 scratch-block padding of graph inputs (nanovllm/engine/model_runner.py:
 842-869, :1154) and the LM head's last-row selection
 (nanovllm/layers/embed_head.py:56-71)."""
+import contextlib
+
 import torch
 
-from nanovllm_amd.engine.graph_runner import default_buckets, pad_decode_inputs
+from nanovllm_amd import _native
+from nanovllm_amd.engine.graph_runner import (DecodeGraphRunner, default_buckets,
+                                              pad_decode_inputs)
 from nanovllm_amd.utils.context import Context, last_row_indices
 
 
@@ -37,3 +41,30 @@ def test_last_row_indices_mixed_prefill_and_decode():
     pre = Context(is_prefill=True, cu_seqlens_q=cu)
     assert last_row_indices(pre).tolist() == [3, 4, 8]
     assert last_row_indices(Context()) is None
+
+
+def _runner_and_inputs(bs=3):
+    pool = torch.zeros(4, 64, 2, 128, dtype=torch.bfloat16)
+    runner = DecodeGraphRunner([pool], [pool], 4, max_bs=4, max_blocks_per_seq=2, scale=1.0)
+    rows = [torch.ones(1, bs, h, 128, dtype=torch.bfloat16) for h in (4, 2, 2)]
+    ints = torch.arange(bs, dtype=torch.int32)
+    return runner, (*rows, ints, ints + 1, torch.zeros(bs, 2, dtype=torch.int32))
+
+
+def test_staging_launch_runs_on_the_pools_device(monkeypatch):
+    # The launch takes a raw stream handle, and a default stream's handle names
+    # the current device's stream, so the pool's device is made current.
+    runner, inputs = _runner_and_inputs()
+    current, launched = [], []
+
+    @contextlib.contextmanager
+    def device(d):
+        current.append(d)
+        yield
+        current.pop()
+
+    monkeypatch.setattr(torch.cuda, "device", device)
+    monkeypatch.setattr(_native, "stream_of", lambda t: 0)
+    monkeypatch.setattr(_native, "call", lambda name, *a: launched.append((name, list(current))))
+    runner._stage(3, 4, *inputs)
+    assert launched == [("kvc_stage_decode", [runner.q.device])] and not current
