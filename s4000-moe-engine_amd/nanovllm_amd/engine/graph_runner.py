@@ -143,7 +143,10 @@ class DecodeGraphRunner:
     def _stageable(self, bs: int, q, k, v, slot_mapping, context_lens, block_tables) -> bool:
         """Inputs the staging launch reads as they are: bf16 rows whose heads
         are dense and 16-byte aligned, int32 / int64 vectors, int32 tables,
-        all on the runner's device."""
+        all plain tensors on the runner's device."""
+        if any(type(t) not in (torch.Tensor, torch.nn.Parameter)
+               for t in (q, k, v, slot_mapping, context_lens, block_tables)):
+            return False
         for t, buf in ((q, self.q), (k, self.k), (v, self.v)):
             if t.dtype != buf.dtype or t.device != buf.device or t.dim() != 4 \
                     or t.size(0) != buf.size(0) or t.size(1) != bs or t.shape[2:] != buf.shape[2:] \

@@ -68,3 +68,13 @@ def test_staging_launch_runs_on_the_pools_device(monkeypatch):
     monkeypatch.setattr(_native, "call", lambda name, *a: launched.append((name, list(current))))
     runner._stage(3, 4, *inputs)
     assert launched == [("kvc_stage_decode", [runner.q.device])] and not current
+
+
+def test_tensor_subclasses_are_staged_by_torch_operators():
+    # A subclass may have no storage to read; its operators know how to copy it.
+    runner, inputs = _runner_and_inputs()
+    assert runner._stageable(3, *inputs)
+    plain = type("Wrapped", (torch.Tensor,), {})
+    for i in range(len(inputs)):
+        mixed = [t.as_subclass(plain) if i == j else t for j, t in enumerate(inputs)]
+        assert not runner._stageable(3, *mixed)
