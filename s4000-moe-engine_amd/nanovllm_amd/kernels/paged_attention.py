@@ -189,6 +189,11 @@ def decode_append_into(output, q, key, value, k_cache, v_cache, slot_mapping, bl
             "GQA-divisible heads")
     if not (q.dtype == key.dtype == value.dtype == k_cache.dtype == torch.bfloat16):
         raise ValueError("paged_decode_append takes a bf16 pool and bf16 q/k/v")
+    if output is not None:
+        if output.shape != q.shape or output.dtype != q.dtype or output.device != q.device:
+            raise ValueError("output must be bf16 [batch, heads, 128] on q's device")
+        if output.stride(2) != 1:
+            raise AssertionError("output needs a unit inner stride")
     assert key.size(0) == batch and key.size(1) == num_kv_heads and slot_mapping.numel() == batch
     assert key.stride(-1) == 1 and value.stride(-1) == 1
     nat.require_device(q, key, value, k_cache, v_cache, slot_mapping, block_tables, context_lens)

@@ -5,7 +5,8 @@ import pytest
 import torch
 
 from nanovllm_amd import _native as nat
-from nanovllm_amd.kernels.paged_attention import paged_decode_append, paged_decode_attention
+from nanovllm_amd.kernels.paged_attention import (decode_append_into, paged_decode_append,
+                                                  paged_decode_attention)
 from nanovllm_amd.layers.rotary import build_cos_sin_cache, qk_norm_rope_store
 
 pytestmark = pytest.mark.gpu
@@ -206,3 +207,27 @@ def test_rope_refuses_a_v_pool_alone():
         qk_norm_rope_store(q, k, v, pos, cs, v_cache=pool, slot_mapping=pos.int())
     with pytest.raises(ValueError, match="v_cache"):
         qk_norm_rope_store(q, k, v, pos, cs, k_cache=pool, slot_mapping=pos.int())
+
+
+@pytest.mark.parametrize("heads,kvh,batch", [(32, 4, 5), (16, 2, 1), (16, 8, 3), (6, 1, 2)])
+@pytest.mark.parametrize("view", [False, True])
+def test_decode_into_a_given_output(monkeypatch, heads, kvh, batch, view):
+    print(f"[host] decode into output {heads}/{kvh} batch {batch} view={view}", flush=True)
+
+    def make():
+        a = _step(heads, kvh, batch, "views")
+        out = torch.full((batch + 1, heads + 2, 128), 7.0, dtype=torch.bfloat16, device=DEV)
+        given = out[:batch, 1:heads + 1] if view else out[:batch, :heads].contiguous()
+        return (given, a["q"], a["k"], a["v"], a["kc"], a["vc"], a["slots"], a["bt"], a["lens"],
+                a["scale"]), [out, a["kc"], a["vc"]]
+
+    (native, python), served = _calls(monkeypatch, decode_append_into, make)
+    assert served
+    assert _same(native[0], python[0]) and _same(native[1], python[1])
+    args, kept = make()
+    assert decode_append_into(*args) is args[0]
+    want = paged_decode_append(*make()[0][1:])
+    assert torch.equal(args[0], want)
+    if view:                                   # nothing around the view is written
+        kept[0][:batch, 1:heads + 1] = 7.0
+        assert bool((kept[0] == 7.0).all())

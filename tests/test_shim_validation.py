@@ -6,7 +6,7 @@ import torch
 
 from nanovllm_amd.engine.kv_offload import HostBlockPool
 from nanovllm_amd.engine.offload_pipeline import AsyncOffloader
-from nanovllm_amd.kernels.paged_attention import paged_decode_append
+from nanovllm_amd.kernels.paged_attention import decode_append_into, paged_decode_append
 
 
 def _decode_args(head_dim=128, page=256, dtype=torch.bfloat16, heads=32, kvh=4):
@@ -27,6 +27,20 @@ def test_paged_decode_append_rejects_unsupported_shapes(bad):
 def test_paged_decode_append_needs_device_tensors():
     with pytest.raises(RuntimeError, match="device"):
         paged_decode_append(*_decode_args())
+
+
+@pytest.mark.parametrize("bad", [
+    lambda q: q[:1].clone(),                                  # fewer rows
+    lambda q: q[:, :16].clone(),                              # fewer heads
+    lambda q: q.flatten(1),                                   # another rank
+    lambda q: q.float(),                                      # another type
+    lambda q: q.to("meta"),                                   # another device
+    lambda q: torch.zeros(2, 32, 256, dtype=q.dtype)[..., ::2],  # dims apart
+])
+def test_decode_append_into_checks_the_given_output(bad):
+    q, *rest = _decode_args()
+    with pytest.raises((ValueError, AssertionError), match="output"):
+        decode_append_into(bad(q), q, *rest)
 
 
 def test_async_offloader_validates_before_the_device():
