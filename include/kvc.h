@@ -556,9 +556,12 @@ int kvc_qk_norm_rope_store(const void* q, int64_t q_stride_t, int64_t q_stride_h
  * r*row_stride, bytes, all multiples of 16 and 16-byte aligned) goes to row r
  * of the dense [layers][dst_rows] destination; rows batch .. bucket - 1 are
  * zeroed.  slots_dst / lens_dst [bucket] take slot_mapping / context_lens
- * (int32 or int64 by index bytes), then scratch_slot / 1; row r of tables_dst
- * [dst_rows, dst_cols] takes block_tables' bt_cols entries (row stride
- * bt_stride elements), everything else scratch_block. */
+ * (int32 or int64 by index bytes), then scratch_slot / 1; row r < batch of
+ * tables_dst [dst_rows, dst_cols] takes block_tables' bt_cols entries (row
+ * stride bt_stride elements) and scratch_block past them, rows batch ..
+ * bucket - 1 scratch_block alone.  Rows bucket .. dst_rows - 1 of every
+ * destination keep what they hold.  slot_mapping and context_lens may be null
+ * when batch is 0, block_tables also when bt_cols is 0. */
 int kvc_stage_decode(const void* q, int64_t q_layer_stride, int64_t q_row_stride, const void* k,
                      int64_t k_layer_stride, int64_t k_row_stride, const void* v,
                      int64_t v_layer_stride, int64_t v_row_stride, int64_t q_row_bytes,

@@ -101,6 +101,11 @@ extern "C" int kvc_stage_decode(const void* q, int64_t q_layer_stride, int64_t q
   KVC_REQUIRE((slot_index_bytes == 4 || slot_index_bytes == 8) &&
                   (lens_index_bytes == 4 || lens_index_bytes == 8),
               KVC_ERR_VALUE, "stage_decode: indices are int32 or int64");
+  KVC_REQUIRE(slots_dst != nullptr && lens_dst != nullptr &&
+                  (tables_dst != nullptr || dst_cols == 0) &&
+                  (batch == 0 || (slot_mapping != nullptr && context_lens != nullptr)) &&
+                  (batch == 0 || bt_cols == 0 || block_tables != nullptr),
+              KVC_ERR_VALUE, "stage_decode: null slots, lengths or tables");
   const void* ptrs[] = {q, k, v, q_dst, k_dst, v_dst};
   for (const void* p : ptrs)
     KVC_REQUIRE(p != nullptr && reinterpret_cast<uintptr_t>(p) % 16 == 0, KVC_ERR_ASSERT,

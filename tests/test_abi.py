@@ -159,6 +159,28 @@ def test_fresh_rows_with_outlier_dims_are_checked_on_the_host():
         call(out_idx2d=None)
 
 
+def test_stage_decode_checks_its_arguments_on_the_host():
+    import pytest
+    # Fake pointers are never dereferenced: a check fails first (without a GPU
+    # a call that passes the checks fails at its launch, RuntimeError).
+
+    def stage(q=64, slots=64, lens=64, tables=64, slots_dst=64, lens_dst=64, tables_dst=64,
+              batch=1, cols=1, dst_cols=2, bytes_=4):
+        _native.call("kvc_stage_decode", q, 256, 256, 64, 256, 256, 64, 256, 256, 256, 256, 1,
+                     batch, 2, 2, slots, bytes_, lens, 4, tables, cols, cols, 64, 64, 64, slots_dst,
+                     lens_dst, tables_dst, dst_cols, 0, 0, None)
+
+    for name in ("slots", "lens", "tables", "slots_dst", "lens_dst", "tables_dst"):
+        with pytest.raises(ValueError, match="null"):
+            stage(**{name: None})
+    with pytest.raises(ValueError, match="shape"):
+        stage(cols=3)
+    with pytest.raises(ValueError, match="int32 or int64"):
+        stage(bytes_=2)
+    with pytest.raises(AssertionError, match="aligned"):
+        stage(q=72)
+
+
 def test_side_pool_widths_and_alignment():
     import pytest
     # Per-channel side pools (kv_dtype 2): n_out_max must be 1, 2, 4 or 8 and
