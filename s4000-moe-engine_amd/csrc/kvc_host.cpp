@@ -15,6 +15,7 @@
 #include <ATen/ATen.h>
 #include <dlfcn.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/version.h>
 
 #include <cstdlib>
 #include <cstring>
@@ -326,4 +327,11 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_kvc_host", nullptr, -1, methods,
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__kvc_host() { return PyModule_Create(&module); }
+PyMODINIT_FUNC PyInit__kvc_host() {
+  PyObject* m = PyModule_Create(&module);
+  if (m != nullptr && PyModule_AddStringConstant(m, "torch_version", TORCH_VERSION) < 0) {
+    Py_DECREF(m);
+    return nullptr;
+  }
+  return m;
+}

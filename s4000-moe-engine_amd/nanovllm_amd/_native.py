@@ -14,6 +14,7 @@ import importlib.util
 import os
 import pathlib
 import threading
+import warnings
 
 import torch
 
@@ -135,27 +136,50 @@ def load() -> ctypes.CDLL:
     return _lib
 
 
+class _NoHostPath:
+    """Stands in for an extension that cannot be loaded: declines every call,
+    and the Python functions make them (the same launches, 5-13 us more host
+    time a decode step)."""
+    decode = staticmethod(lambda *_: None)
+    rope = staticmethod(lambda *_: None)
+
+
 _host = None
 
 
+def load_host():
+    """The native host path of the decode step (csrc/kvc_host.cpp), bound to
+    libkvc; RuntimeError when it is absent, does not load or was built for
+    another torch."""
+    load()
+    try:
+        loader = importlib.machinery.ExtensionFileLoader("_kvc_host", str(HOST_PATH))
+        spec = importlib.util.spec_from_file_location("_kvc_host", str(HOST_PATH), loader=loader)
+        module = importlib.util.module_from_spec(spec)
+        loader.exec_module(module)
+    except (ImportError, OSError) as e:
+        raise RuntimeError(f"{HOST_PATH} does not load ({e}); build it with "
+                           f"`make -C {PKG_ROOT / 'csrc'}`") from e
+    if not torch.__version__.startswith(module.torch_version):
+        raise RuntimeError(f"{HOST_PATH} was built for torch {module.torch_version}, this is "
+                           f"{torch.__version__}; build it with `make -C {PKG_ROOT / 'csrc'}`")
+    module.bind(str(LIB_PATH))
+    return module
+
+
 def host():
-    """The native host path of the decode step (csrc/kvc_host.cpp), loaded
-    once and bound to libkvc; RuntimeError when it is absent."""
+    """The native host path, loaded once.  Without it a warning is given and
+    the Python path makes every call."""
     global _host
     if _host is None:
         load()
         with _lock:
             if _host is None:
-                if not HOST_PATH.is_file():
-                    raise RuntimeError(f"_kvc_host.so not found at {HOST_PATH}; build it with "
-                                       f"`make -C {PKG_ROOT / 'csrc'}`")
-                loader = importlib.machinery.ExtensionFileLoader("_kvc_host", str(HOST_PATH))
-                spec = importlib.util.spec_from_file_location("_kvc_host", str(HOST_PATH),
-                                                              loader=loader)
-                module = importlib.util.module_from_spec(spec)
-                loader.exec_module(module)
-                module.bind(str(LIB_PATH))
-                _host = module
+                try:
+                    _host = load_host()
+                except RuntimeError as e:
+                    warnings.warn(f"no native host path: {e}", RuntimeWarning, stacklevel=3)
+                    _host = _NoHostPath
     return _host
 
 

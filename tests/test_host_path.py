@@ -1,11 +1,14 @@
-"""The native host path (csrc/kvc_host.cpp) on calls that it cannot serve, on
-the CPU: arguments without storage that pass for GPU tensors.  Each case runs
-in a process of its own, since what it guards against ends the process."""
+"""The native host path (csrc/kvc_host.cpp) where it cannot serve, on the
+CPU: arguments without storage that pass for GPU tensors (each case in a
+process of its own, since what it guards against ends the process), and an
+extension that is absent or does not load."""
 import pathlib
 import subprocess
 import sys
+import warnings
 
 import pytest
+import torch
 
 from nanovllm_amd import _native
 
@@ -66,3 +69,23 @@ def test_tensors_without_storage_are_refused(call):
                          cwd=pathlib.Path(__file__).parent)
     assert run.returncode == 0, (run.returncode, run.stderr[-2000:])
     assert run.stdout.strip() == "refused [None]"
+
+
+@pytest.mark.parametrize("broken", ["absent", "not a library", "another torch"])
+def test_calls_take_the_python_path_without_the_extension(monkeypatch, tmp_path, broken):
+    path = tmp_path / "_kvc_host.so"
+    if broken == "not a library":
+        path.write_bytes(b"not ELF")
+    elif broken == "another torch":
+        path = _native.HOST_PATH
+        monkeypatch.setattr(torch, "__version__", "1.0.0")
+    monkeypatch.setattr(_native, "HOST_PATH", path)
+    monkeypatch.setattr(_native, "_host", None)
+    with pytest.warns(RuntimeWarning, match="host path"):
+        host = _native.host()
+    assert host.decode(*range(11)) is None and host.rope(*range(13)) is None
+    with warnings.catch_warnings():           # said once
+        warnings.simplefilter("error")
+        assert _native.host() is host
+    with pytest.raises(RuntimeError):
+        _native.load_host()
