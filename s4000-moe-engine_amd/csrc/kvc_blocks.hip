@@ -60,8 +60,9 @@ __device__ __forceinline__ void select_blocks(const MoveArgs& a, const InlineIds
   d = a.dst_ids ? int64_t(ids.dst[item]) : item;
 }
 
-// One 16 KiB piece of one row (item, plane).
-template <bool kStream>
+// One 16 KiB piece of one row (item, plane), with non-temporal loads and / or
+// stores.
+template <bool kStreamLoads, bool kStreamStores>
 __device__ __forceinline__ void move_piece(const MoveArgs& a, int64_t s_sel, int64_t d_sel,
                                            int64_t plane, int64_t piece) {
   const char* s = a.src + plane * a.src_plane + s_sel * a.src_item + piece * kPiece;
@@ -73,14 +74,14 @@ __device__ __forceinline__ void move_piece(const MoveArgs& a, int64_t s_sel, int
     const int64_t off = (int64_t(u) * kThreads + threadIdx.x) * 16;
     if (off >= limit) continue;
     const u32x4_t* from = reinterpret_cast<const u32x4_t*>(s + off);
-    v[u] = kStream ? __builtin_nontemporal_load(from) : *from;
+    v[u] = kStreamLoads ? __builtin_nontemporal_load(from) : *from;
   }
 #pragma unroll
   for (int u = 0; u < kUnroll; ++u) {
     const int64_t off = (int64_t(u) * kThreads + threadIdx.x) * 16;
     if (off >= limit) continue;
     u32x4_t* to = reinterpret_cast<u32x4_t*>(d + off);
-    if (kStream) {
+    if (kStreamStores) {
       __builtin_nontemporal_store(v[u], to);
     } else {
       *to = v[u];
@@ -91,15 +92,31 @@ __device__ __forceinline__ void move_piece(const MoveArgs& a, int64_t s_sel, int
 // In-HBM move, bound by HBM: every byte is read once and written once.
 // Workgroup b runs on XCD b mod 8; it takes piece (b mod 8) * per + b / 8, so
 // one XCD's workgroups walk one contiguous run of pieces (and its memory
-// channels see long runs), and loads and stores bypass the caches' reuse
-// order.  16 blocks of 24 MiB (805 MB moved): 155 us with pieces in launch
-// order and plain accesses, 147 us with the XCD order alone, 145 us with
-// non-temporal accesses alone, 134 us (6.0 TB/s) with both; 32 KiB pieces
-// and 1024-thread workgroups 134-137 us; persistent grids 149-160 us (copies
-// alone; the whole BlockMover.copy call, then still uploading its ids, went
-// from 165 to 148-150 us).
+// channels see long runs), and loads are non-temporal.  16 blocks of 24 MiB
+// (805 MB moved): 155 us with pieces in launch order and plain accesses, 147
+// us with the XCD order alone, 145 us with non-temporal accesses alone, 134
+// us (6.0 TB/s) with both; 32 KiB pieces and 1024-thread workgroups 134-137
+// us; persistent grids 149-160 us (copies alone; the whole BlockMover.copy
+// call, then still uploading its ids, went from 165 to 148-150 us).
+//
+// kStreamStores (kStreamStoreBytes and more): what a smaller move writes fits
+// the 256 MB memory-side cache, and plain stores leave it there for its reader
+// (the next decode step, the wire, a DMA).  us of a gather of blocks that no
+// cache holds, and of the gather with a reduction over its result, for both
+// accesses plain in launch order / both non-temporal / this rule's form:
+//      8 MB   6.6  5.9  6.0     18.6  19.4  18.5
+//     25 MB  13.9 11.5 12.4     28.3  28.9  27.7
+//     50 MB  24.4 20.6 22.3     41.4  43.7  39.7
+//    101 MB  44.4 38.0 41.4     71.6  72.5  62.0
+//    201 MB  83.3 71.4 77.7    133.8 130.3 123.2
+//    252 MB 102.6 89.5 98.1    165.7 160.7 142.1
+//    403 MB   162  139  151      260   247   246 (plain stores; above the line)
+// Blocks that the cache already holds move faster with plain loads (25 MB: 8.1
+// against 10.1 us, 67 MB: 18 against 24 us; from 75 MB on 31 against 27 us);
+// a compaction's or an export's blocks are not such blocks.
 // `total` < 2^31, so 32-bit divisions do.
-template <typename Ids>
+constexpr int64_t kStreamStoreBytes = int64_t(256) << 20;
+template <bool kStreamStores, typename Ids>
 __global__ void __launch_bounds__(kThreads)
 move_blocks_kernel(MoveArgs a, uint32_t total, uint32_t per, Ids ids) {
   const uint32_t w = (blockIdx.x & 7u) * per + (blockIdx.x >> 3);
@@ -108,7 +125,8 @@ move_blocks_kernel(MoveArgs a, uint32_t total, uint32_t per, Ids ids) {
   const uint32_t item = row / uint32_t(a.planes);
   int64_t s, d;
   select_blocks(a, ids, item, s, d);
-  move_piece<true>(a, s, d, row - item * uint32_t(a.planes), w - row * uint32_t(a.pieces));
+  move_piece<true, kStreamStores>(a, s, d, row - item * uint32_t(a.planes),
+                                  w - row * uint32_t(a.pieces));
 }
 
 // Moves to or from pinned host memory.
@@ -119,7 +137,7 @@ __global__ void __launch_bounds__(kThreads) move_host_kernel(MoveArgs a, int64_t
     const int64_t item = row / a.planes;
     int64_t s, d;
     select_blocks(a, ids, item, s, d);
-    move_piece<false>(a, s, d, row - item * a.planes, w - row * a.pieces);
+    move_piece<false, false>(a, s, d, row - item * a.planes, w - row * a.pieces);
   }
 }
 
@@ -134,7 +152,7 @@ int64_t host_move_workgroups() {
 
 template <typename Ids>
 int launch_one(const MoveArgs& a, int64_t n, hipStream_t st, const char* what, bool host_side,
-               const Ids& ids) {
+               bool stream_stores, const Ids& ids) {
   const int64_t total = n * a.planes * a.pieces;
   if (host_side) {
     const int64_t grid = std::min(total, host_move_workgroups());
@@ -146,7 +164,11 @@ int launch_one(const MoveArgs& a, int64_t n, hipStream_t st, const char* what, b
   KVC_REQUIRE(total < (int64_t(1) << 31), KVC_ERR_VALUE, "%s: %lld workgroups exceed one launch",
               what, (long long)total);
   const uint32_t per = uint32_t((total + 7) / 8);
-  move_blocks_kernel<<<8 * per, kThreads, 0, st>>>(a, uint32_t(total), per, ids);
+  if (stream_stores) {
+    move_blocks_kernel<true><<<8 * per, kThreads, 0, st>>>(a, uint32_t(total), per, ids);
+  } else {
+    move_blocks_kernel<false><<<8 * per, kThreads, 0, st>>>(a, uint32_t(total), per, ids);
+  }
   return check_launch(what);
 }
 
@@ -155,7 +177,8 @@ int launch_one(const MoveArgs& a, int64_t n, hipStream_t st, const char* what, b
 int launch_move(const MoveArgs& a, int64_t n, hipStream_t st, const char* what,
                 bool host_side = false, bool ids_on_host = false) {
   if (n == 0 || a.planes == 0 || a.block_bytes == 0) return KVC_OK;
-  if (!ids_on_host) return launch_one(a, n, st, what, host_side, DeviceIds{});
+  const bool stream_stores = n * a.planes * a.block_bytes >= kStreamStoreBytes;
+  if (!ids_on_host) return launch_one(a, n, st, what, host_side, stream_stores, DeviceIds{});
   for (int64_t i0 = 0; i0 < n; i0 += kInlineIds) {
     const int64_t m = std::min<int64_t>(kInlineIds, n - i0);
     InlineIds ids;
@@ -170,7 +193,7 @@ int launch_move(const MoveArgs& a, int64_t n, hipStream_t st, const char* what,
     } else {
       part.dst = a.dst + i0 * a.dst_item;
     }
-    const int rc = launch_one(part, m, st, what, host_side, ids);
+    const int rc = launch_one(part, m, st, what, host_side, stream_stores, ids);
     if (rc != KVC_OK) return rc;
   }
   return KVC_OK;

@@ -147,3 +147,27 @@ def test_device_moves_at_piece_and_xcd_edges(planes, row_bytes, n):
     expect[:, :, src] = items.movedim(0, 2)
     mover.scatter(host, src)
     assert torch.equal(pool, expect)
+
+
+@pytest.mark.parametrize("planes,row_bytes,n", [
+    (2, 16 << 20, 7),      # 224 MiB: plain stores
+    (2, 16 << 20, 8),      # 256 MiB: non-temporal stores
+    (1, 1 << 20, 255), (1, 1 << 20, 257),  # the same line; 257 ids take two launches
+])
+def test_device_moves_around_the_streaming_store_size(planes, row_bytes, n):
+    g = torch.Generator(device=DEV).manual_seed(3)
+    pool = torch.randint(0, 1 << 62, (1, planes, 2 * n + 1, row_bytes // 8), generator=g,
+                         dtype=torch.int64, device=DEV)
+    ids = torch.randperm(2 * n + 1, generator=torch.Generator().manual_seed(3)).tolist()
+    src, dst = ids[:n], ids[n:2 * n]
+    mover = BlockMover(pool)
+    expect = pool.clone()
+    print(f"[blocks] streaming stores planes={planes} row={row_bytes} n={n}", flush=True)
+    items = mover.gather(src)
+    assert torch.equal(items, expect[:, :, src].movedim(2, 0))
+    expect[:, :, dst] = expect[:, :, src]
+    mover.copy(src, dst)
+    assert torch.equal(pool, expect)
+    expect[:, :, src] = items.movedim(0, 2).flip(2)
+    mover.scatter(items.flip(0).contiguous(), torch.tensor(src, device=DEV))
+    assert torch.equal(pool, expect)
