@@ -4,6 +4,7 @@ import numpy as np
 import pytest
 import torch
 
+from nanovllm_amd import _native as nat
 from nanovllm_amd.engine.kv_runner import BlockMover
 from oracle import kv_oracle as ko
 
@@ -171,3 +172,33 @@ def test_device_moves_around_the_streaming_store_size(planes, row_bytes, n):
     expect[:, :, src] = items.movedim(0, 2).flip(2)
     mover.scatter(items.flip(0).contiguous(), torch.tensor(src, device=DEV))
     assert torch.equal(pool, expect)
+
+
+@pytest.mark.parametrize("n,inline", [(256, (True, True)), (257, (False, True)),
+                                      (512, (False, True)), (513, (False, False))])
+def test_id_lists_go_with_the_launch_or_are_uploaded(monkeypatch, n, inline):
+    # A gather / scatter list of up to 256 ids and a copy's lists of up to 512
+    # go with the launches; a host tensor does at any length.
+    pool = torch.arange(2 * n, dtype=torch.int64, device=DEV).view(1, 1, -1, 1).repeat(1, 2, 1, 2)
+    mover, called = BlockMover(pool), []
+    real = nat.call
+    monkeypatch.setattr(nat, "call", lambda name, *a: (called.append(name), real(name, *a))[1])
+    ids = torch.randperm(2 * n, generator=torch.Generator().manual_seed(n)).tolist()
+    src, dst = ids[:n], ids[n:]
+    print(f"[blocks] id lists n={n}", flush=True)
+    items = mover.gather(src)
+    assert torch.equal(mover.gather(torch.tensor(src)), items)
+    host = torch.empty(items.shape, dtype=items.dtype, pin_memory=True)
+    mover.gather(src, out=host)
+    expect = pool.clone()
+    expect[:, :, dst] = expect[:, :, src]
+    assert torch.equal(items, expect[:, :, dst].movedim(2, 0))
+    mover.copy(src, dst)
+    assert torch.equal(pool, expect) and torch.equal(host, items.cpu())
+    mover.scatter(items.flip(0).contiguous(), src)
+    expect[:, :, src] = items.flip(0).movedim(0, 2)
+    assert torch.equal(pool, expect)
+    form = ["_ids" if i else "" for i in inline]
+    assert called == ["kvc_block_gather" + form[0], "kvc_block_gather_ids",
+                      "kvc_block_gather" + form[0], "kvc_block_copy" + form[1],
+                      "kvc_block_scatter" + form[0]]
