@@ -99,25 +99,24 @@ __device__ __forceinline__ void move_piece(const MoveArgs& a, int64_t s_sel, int
 // us; persistent grids 149-160 us (copies alone; the whole BlockMover.copy
 // call, then still uploading its ids, went from 165 to 148-150 us).
 //
-// kStreamStores (kStreamStoreBytes and more): what a smaller move writes fits
-// the 256 MB memory-side cache, and plain stores leave it there for its reader
-// (the next decode step, the wire, a DMA).  us of a gather of blocks that no
-// cache holds, and of the gather with a reduction over its result, for both
-// accesses plain in launch order / both non-temporal / this rule's form:
-//      8 MB   6.6  5.9  6.0     18.6  19.4  18.5
-//     25 MB  13.9 11.5 12.4     28.3  28.9  27.7
-//     50 MB  24.4 20.6 22.3     41.4  43.7  39.7
-//    101 MB  44.4 38.0 41.4     71.6  72.5  62.0
-//    201 MB  83.3 71.4 77.7    133.8 130.3 123.2
-//    252 MB 102.6 89.5 98.1    165.7 160.7 142.1
-//    403 MB   162  139  151      260   247   246 (plain stores; above the line)
-// A scatter of items just written, with a reduction over the blocks: 25 MB 55.4
-// 56.7 51.1, 101 MB 156 183 138, 201 MB 356 349 250.
-// Blocks that the cache already holds move faster with plain loads (25 MB: 8.1
-// against 10.1 us, 67 MB: 18 against 24 us; from 75 MB on 31 against 27 us);
-// a compaction's or an export's blocks are not such blocks.
+// kStreamStores (from kStreamStoreBytes on): plain stores leave what is written
+// in the memory-side cache for its reader, non-temporal ones make a large move
+// itself shorter.  us of a gather of blocks that no cache holds, alone and with
+// a reduction over its result, for accesses plain in launch order /
+// non-temporal loads and stores / non-temporal loads only:
+//      8 MB   6.7   6.1   6.1     18.9  20.0  18.6
+//     13 MB   7.8   7.5   7.1     20.9  22.1  20.7
+//     17 MB   9.6   8.2   8.3     23.3  23.5  22.4
+//     25 MB  13.9  11.5  12.4     28.3  28.9  27.7
+//    101 MB  44.4  38.0  41.4     71.6  72.5  62.0
+//    252 MB 102.6  89.5  98.1    165.7 160.7 142.1
+//    403 MB   162   139   151      260   247   246
+// Up to 16 MiB the loads alone are worth as much as both; past it a move alone
+// gains up to 10 % from the stores, which a reader right behind it loses
+// again; blocks that are moved are mostly read much later.  Blocks that a cache
+// already holds move faster with plain accesses (25 MB: 8.1 against 10.4 us).
 // `total` < 2^31, so 32-bit divisions do.
-constexpr int64_t kStreamStoreBytes = int64_t(256) << 20;
+constexpr int64_t kStreamStoreBytes = int64_t(16) << 20;
 template <bool kStreamStores, typename Ids>
 __global__ void __launch_bounds__(kThreads)
 move_blocks_kernel(MoveArgs a, uint32_t total, uint32_t per, Ids ids) {

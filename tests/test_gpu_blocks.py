@@ -151,9 +151,10 @@ def test_device_moves_at_piece_and_xcd_edges(planes, row_bytes, n):
 
 
 @pytest.mark.parametrize("planes,row_bytes,n", [
-    (2, 16 << 20, 7),      # 224 MiB: plain stores
-    (2, 16 << 20, 8),      # 256 MiB: non-temporal stores
-    (1, 1 << 20, 255), (1, 1 << 20, 257),  # the same line; 257 ids take two launches
+    (2, 1 << 20, 7),       # 14 MiB: plain stores
+    (2, 1 << 20, 8),       # 16 MiB: non-temporal stores
+    (1, 1 << 16, 255), (1, 1 << 16, 256),
+    (1, 16 << 20, 17),     # past the memory-side cache
 ])
 def test_device_moves_around_the_streaming_store_size(planes, row_bytes, n):
     g = torch.Generator(device=DEV).manual_seed(3)
