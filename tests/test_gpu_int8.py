@@ -108,6 +108,36 @@ def test_chan_store_matches_p17_unit_bitwise():
         assert np.array_equal(a, b), f"{name} differs"
 
 
+@pytest.mark.parametrize("nout", [1, 3, 8, 9, 15, 16])
+@pytest.mark.parametrize("tokens", [1, 5, 130])
+def test_chan_store_at_every_side_width_bitwise(nout, tokens):
+    # The append takes side widths up to 16 (a lane of a row's 16 per outlier
+    # dim); heads with all, none, all but one and half of the slots in use.
+    # Every byte of the pools is compared, slots that no token writes included.
+    KVH, D, blocks = 4, 128, 2
+    print(f"[int8-chan] store width {nout} tokens {tokens}", flush=True)
+    g = torch.Generator().manual_seed(100 * nout + tokens)
+    key, value = (torch.randn(tokens, KVH, D, generator=g).mul_(5).to(torch.bfloat16)
+                  for _ in range(2))
+    s_k, s_v = (torch.rand(KVH, D, generator=g).add_(0.5).mul_(0.05) for _ in range(2))
+    n_out = torch.tensor([nout, 0, nout - 1, nout // 2], dtype=torch.int32)
+    dims = torch.stack([torch.randperm(D, generator=g)[:nout] for _ in range(KVH)]).int()
+    slot = torch.randperm(blocks * 256, generator=g)[:tokens].int()
+    codes = [torch.randint(-127, 128, (blocks, 256, KVH, D), generator=g, dtype=torch.int8)
+             for _ in range(2)]
+    sides = [torch.randn(blocks, 256, KVH, nout, generator=g).to(torch.bfloat16) for _ in range(2)]
+    got = [t.to(DEV) for t in (*codes, *sides)]
+    store_kvcache_int8(key.to(DEV), value.to(DEV), got[0], got[1], s_k.to(DEV), s_v.to(DEV),
+                       got[2], got[3], dims.to(DEV), n_out.to(DEV), slot.to(DEV))
+    torch.cuda.synchronize()
+    want = [codes[0].numpy(), codes[1].numpy(), bits(sides[0]), bits(sides[1])]
+    ko.store_int8_chan(bits(key), bits(value), want[0], want[1], s_k.numpy(), s_v.numpy(), want[2],
+                       want[3], dims.numpy(), n_out.numpy(), slot.numpy())
+    for name, a, b in zip(("k codes", "v codes", "k side", "v side"), got, want):
+        a = a.cpu().numpy() if a.dtype == torch.int8 else bits(a)
+        assert np.array_equal(a, b), f"{name} differ"
+
+
 def test_chan_store_strided_v():
     # The reference kernel reads V with K's strides; this path takes V's own.
     key, value, s_k, s_v, _, _, out_idx2d, head_n_out = p17_unit_inputs()
