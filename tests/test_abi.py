@@ -254,8 +254,8 @@ def test_mixed_split_from_the_work_hints(monkeypatch):
 
 
 def test_host_extension_has_no_thread_local_storage():
-    # A TLS segment in a library loaded after startup slows every later TLS
-    # access of the process (see the Makefile).
+    # A TLS segment that no thread touches, in a library loaded after startup,
+    # slows every other TLS access of the process (see the Makefile).
     import struct
     data = _native.HOST_PATH.read_bytes()
     assert data[:6] == b"\x7fELF\x02\x01"
