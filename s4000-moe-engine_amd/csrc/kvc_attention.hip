@@ -3946,9 +3946,18 @@ __device__ __forceinline__ void p2_load_chunk(PfItem& it, const int4* ctab, cons
 #endif
 constexpr int kP2ItemCost = KVC_P2_ITEM_COST;
 // With the residue product an item also reads its outlier dims' list and
-// folds the residues in at its end: four chunks of 300-512 tokens after
-// 0-8192 keys took 196 / 191 / 187.4 / 186.1 / 185.5 / 186.4 us a call at
-// 6 / 7 / 8 / 9 / 10 / 12.
+// folds the residues in at its end.  us a call (store, gather and merge
+// included) at 6 / 8 / 10 / 12:
+//   32 q / 4 kv heads, 4 chunks of 300-512 tokens after 0-8192  198 190 188 187
+//     4 of 1000-1024 after 0-4096                             310 283 281 277
+//     12 of 100-507 after 0-2321                              246 228 225 223
+//     6 of 17-200 after 0-2000                               61.9 61.9 61.7 62.8
+//     2048 after 4096 / 1024 after 14336      267 267 265 264 / 338 340 337 336
+//   16 / 2, 4 of 300-512 / 2 of 700-1500    118 117 115 114 / 192 169 162 160
+//   16 / 8, 3 of 300-700 after 0-2000                       81.3 78.1 77.6 78.7
+// The cost moves the cuts between shares, and with them the last bits of the
+// split rows (fp16 partials); the distance to 64 bits stays (1.89e-3 ..
+// 1.96e-3 on these at 6 and at 10).
 #ifndef KVC_P2_ITEM_COST_RESIDUE
 #define KVC_P2_ITEM_COST_RESIDUE 10
 #endif
