@@ -474,11 +474,11 @@ int kvc_block_gather(const void* src, int64_t planes, int64_t src_plane_stride,
                      void* dst, int64_t dst_item_stride, int64_t dst_plane_stride,
                      kvc_stream_t stream);
 /* The _ids forms take their block ids from HOST memory (read before the call
- * returns, passed with the launch: no upload). */
+ * returns, passed with the launches, 256 each: no upload). */
 int kvc_block_gather_ids(const void* src, int64_t planes, int64_t src_plane_stride,
-                     int64_t block_bytes, const int32_t* block_ids, int64_t n,
-                     void* dst, int64_t dst_item_stride, int64_t dst_plane_stride,
-                     kvc_stream_t stream);
+                         int64_t block_bytes, const int32_t* block_ids, int64_t n,
+                         void* dst, int64_t dst_item_stride, int64_t dst_plane_stride,
+                         kvc_stream_t stream);
 
 /* Scatter: dst[p][block_ids[i]] = src[i][p].  Replaces the index_copy_ of
  * ModelRunner.offload_get (model_runner.py:300-305) and import_kv
@@ -487,8 +487,8 @@ int kvc_block_scatter(const void* src, int64_t src_item_stride, int64_t src_plan
                       int64_t planes, int64_t block_bytes, const int32_t* block_ids, int64_t n,
                       void* dst, int64_t dst_plane_stride, kvc_stream_t stream);
 int kvc_block_scatter_ids(const void* src, int64_t src_item_stride, int64_t src_plane_stride,
-                      int64_t planes, int64_t block_bytes, const int32_t* block_ids, int64_t n,
-                      void* dst, int64_t dst_plane_stride, kvc_stream_t stream);
+                          int64_t planes, int64_t block_bytes, const int32_t* block_ids, int64_t n,
+                          void* dst, int64_t dst_plane_stride, kvc_stream_t stream);
 
 /* In-HBM copy pool[p][dst_ids[i]] = pool[p][src_ids[i]] (no reference
  * function; the closed form of a compaction step).  The id sets must be
@@ -497,8 +497,8 @@ int kvc_block_copy(void* pool, int64_t planes, int64_t plane_stride, int64_t blo
                    const int32_t* src_ids, const int32_t* dst_ids, int64_t n,
                    kvc_stream_t stream);
 int kvc_block_copy_ids(void* pool, int64_t planes, int64_t plane_stride, int64_t block_bytes,
-                   const int32_t* src_ids, const int32_t* dst_ids, int64_t n,
-                   kvc_stream_t stream);
+                       const int32_t* src_ids, const int32_t* dst_ids, int64_t n,
+                       kvc_stream_t stream);
 
 /* DMA form of the offload byte moves: one strided 2-D copy per block on the
  * copy engines, block ids read from HOST memory (the block manager's ints).

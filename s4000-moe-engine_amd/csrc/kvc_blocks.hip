@@ -249,11 +249,9 @@ int check_geometry(const void* a, const void* b, int64_t planes, int64_t block_b
 using namespace kvc;
 
 namespace {
-int block_gather(const void* src, int64_t planes, int64_t src_plane_stride,
-                                int64_t block_bytes, const int32_t* block_ids, int64_t n,
-                                void* dst, int64_t dst_item_stride, int64_t dst_plane_stride,
-                                kvc_stream_t stream,
-    bool ids_on_host) {
+int block_gather(const void* src, int64_t planes, int64_t src_plane_stride, int64_t block_bytes,
+                 const int32_t* block_ids, int64_t n, void* dst, int64_t dst_item_stride,
+                 int64_t dst_plane_stride, kvc_stream_t stream, bool ids_on_host) {
   clear_error();
   int rc = check_geometry(src, dst, planes, block_bytes,
                           {src_plane_stride, dst_item_stride, dst_plane_stride}, n,
@@ -284,21 +282,22 @@ extern "C" int kvc_block_gather(const void* src, int64_t planes, int64_t src_pla
                                 int64_t block_bytes, const int32_t* block_ids, int64_t n,
                                 void* dst, int64_t dst_item_stride, int64_t dst_plane_stride,
                                 kvc_stream_t stream) {
-  return block_gather(src, planes, src_plane_stride, block_bytes, block_ids, n, dst, dst_item_stride, dst_plane_stride, stream, false);
+  return block_gather(src, planes, src_plane_stride, block_bytes, block_ids, n, dst,
+                      dst_item_stride, dst_plane_stride, stream, false);
 }
+
 extern "C" int kvc_block_gather_ids(const void* src, int64_t planes, int64_t src_plane_stride,
-                                int64_t block_bytes, const int32_t* block_ids, int64_t n,
-                                void* dst, int64_t dst_item_stride, int64_t dst_plane_stride,
-                                kvc_stream_t stream) {
-  return block_gather(src, planes, src_plane_stride, block_bytes, block_ids, n, dst, dst_item_stride, dst_plane_stride, stream, true);
+                                    int64_t block_bytes, const int32_t* block_ids, int64_t n,
+                                    void* dst, int64_t dst_item_stride, int64_t dst_plane_stride,
+                                    kvc_stream_t stream) {
+  return block_gather(src, planes, src_plane_stride, block_bytes, block_ids, n, dst,
+                      dst_item_stride, dst_plane_stride, stream, true);
 }
 
 namespace {
-int block_scatter(const void* src, int64_t src_item_stride,
-                                 int64_t src_plane_stride, int64_t planes, int64_t block_bytes,
-                                 const int32_t* block_ids, int64_t n, void* dst,
-                                 int64_t dst_plane_stride, kvc_stream_t stream,
-    bool ids_on_host) {
+int block_scatter(const void* src, int64_t src_item_stride, int64_t src_plane_stride,
+                  int64_t planes, int64_t block_bytes, const int32_t* block_ids, int64_t n,
+                  void* dst, int64_t dst_plane_stride, kvc_stream_t stream, bool ids_on_host) {
   clear_error();
   int rc = check_geometry(src, dst, planes, block_bytes,
                           {src_item_stride, src_plane_stride, dst_plane_stride}, n,
@@ -329,20 +328,22 @@ extern "C" int kvc_block_scatter(const void* src, int64_t src_item_stride,
                                  int64_t src_plane_stride, int64_t planes, int64_t block_bytes,
                                  const int32_t* block_ids, int64_t n, void* dst,
                                  int64_t dst_plane_stride, kvc_stream_t stream) {
-  return block_scatter(src, src_item_stride, src_plane_stride, planes, block_bytes, block_ids, n, dst, dst_plane_stride, stream, false);
+  return block_scatter(src, src_item_stride, src_plane_stride, planes, block_bytes, block_ids, n,
+                       dst, dst_plane_stride, stream, false);
 }
+
 extern "C" int kvc_block_scatter_ids(const void* src, int64_t src_item_stride,
-                                 int64_t src_plane_stride, int64_t planes, int64_t block_bytes,
-                                 const int32_t* block_ids, int64_t n, void* dst,
-                                 int64_t dst_plane_stride, kvc_stream_t stream) {
-  return block_scatter(src, src_item_stride, src_plane_stride, planes, block_bytes, block_ids, n, dst, dst_plane_stride, stream, true);
+                                     int64_t src_plane_stride, int64_t planes, int64_t block_bytes,
+                                     const int32_t* block_ids, int64_t n, void* dst,
+                                     int64_t dst_plane_stride, kvc_stream_t stream) {
+  return block_scatter(src, src_item_stride, src_plane_stride, planes, block_bytes, block_ids, n,
+                       dst, dst_plane_stride, stream, true);
 }
 
 namespace {
-int block_copy(void* pool, int64_t planes, int64_t plane_stride,
-                              int64_t block_bytes, const int32_t* src_ids, const int32_t* dst_ids,
-                              int64_t n, kvc_stream_t stream,
-    bool ids_on_host) {
+int block_copy(void* pool, int64_t planes, int64_t plane_stride, int64_t block_bytes,
+               const int32_t* src_ids, const int32_t* dst_ids, int64_t n, kvc_stream_t stream,
+               bool ids_on_host) {
   clear_error();
   int rc = check_geometry(pool, pool, planes, block_bytes, {plane_stride}, n, "block_copy");
   if (rc != KVC_OK) return rc;
@@ -369,9 +370,10 @@ extern "C" int kvc_block_copy(void* pool, int64_t planes, int64_t plane_stride,
                               int64_t n, kvc_stream_t stream) {
   return block_copy(pool, planes, plane_stride, block_bytes, src_ids, dst_ids, n, stream, false);
 }
+
 extern "C" int kvc_block_copy_ids(void* pool, int64_t planes, int64_t plane_stride,
-                              int64_t block_bytes, const int32_t* src_ids, const int32_t* dst_ids,
-                              int64_t n, kvc_stream_t stream) {
+                                  int64_t block_bytes, const int32_t* src_ids,
+                                  const int32_t* dst_ids, int64_t n, kvc_stream_t stream) {
   return block_copy(pool, planes, plane_stride, block_bytes, src_ids, dst_ids, n, stream, true);
 }
 
