@@ -231,3 +231,31 @@ def test_decode_into_a_given_output(monkeypatch, heads, kvh, batch, view):
     if view:                                   # nothing around the view is written
         kept[0][:batch, 1:heads + 1] = 7.0
         assert bool((kept[0] == 7.0).all())
+
+
+@pytest.mark.parametrize("call", ["rope", "decode", "append"])
+def test_out_of_memory_is_torchs_error(call):
+    # An allocation that fails before a launch leaves the call to the Python
+    # function, which raises torch's own error; the next call works.
+    # One row repeated: an output of 550 GB, which no card holds.
+    n = 1 << 26
+    q, k, v = (torch.zeros(1, h, 128, dtype=torch.bfloat16, device=DEV).expand(n, h, 128)
+               for h in (32, 4, 4))
+    pool = torch.zeros(1, PAGE, 4, 128, dtype=torch.bfloat16, device=DEV)
+    ints = torch.ones(n, dtype=torch.int32, device=DEV)
+    cs = build_cos_sin_cache(128, 16, 1e6, DEV)
+
+    def run(m):
+        t = ints[:m]
+        if call == "rope":
+            return qk_norm_rope_store(q[:m], k[:m], v[:m], t, cs)
+        if call == "decode":
+            return paged_decode_attention(q[:m], pool, pool, t.view(m, 1) - 1, t, 0.1, 1)
+        return paged_decode_append(q[:m], k[:m], v[:m], pool, pool, t - 1, t.view(m, 1) - 1, t, 0.1)
+
+    run(2)
+    print(f"[host] out of memory: {call}", flush=True)
+    with pytest.raises(torch.OutOfMemoryError):
+        run(n)
+    run(2)
+    torch.cuda.synchronize()
